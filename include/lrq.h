@@ -150,6 +150,24 @@ int lrq_act_qdq(const void* in, int in_dtype, int64_t rows, int64_t cols, int64_
                 unsigned flags, float* out, lrq_stream_t stream);
 
 /*
+ * The FP8 rollout linear for few tokens in one launch:
+ *   out[m, n] = x_dq[m, k] . w_dq[n, k]^T + bias[n]
+ * with x_dq as lrq_act_qdq (blk 128) and w_dq as lrq_fp8_block_dequant (1 x 128
+ * blocks) give them, float32 sums and a result in x's type.  Replaces
+ * _FP8W8A8Linear.forward (lumenrl/quantization/fp8_rollout.py:53-78) on 16-bit
+ * activations.  Sums run in another order than a library product's; an inf or
+ * NaN in a row of x makes that row of out NaN, as the reference's ops do.
+ *   x      : [rows, k] bf16 or fp16, element-aligned, row stride ld >= k;
+ *   codes  : [n, k] e4m3 bytes, dense;  scales : [n, k/128] bf16, dense;
+ *   bias   : [n] of bias_dtype (bf16, fp16 or fp32), or null;
+ *   out    : [rows, n] of x's type, dense, 16-byte aligned.
+ * rows <= 64; k a multiple of 128; k and ld at most 2^24.
+ */
+int lrq_fp8_linear(const void* x, int x_dtype, int64_t rows, int64_t k, int64_t ld,
+                   const uint8_t* codes, const void* scales, int64_t n, const void* bias,
+                   int bias_dtype, void* out, lrq_stream_t stream);
+
+/*
  * Unscaled cast of n contiguous elements to float8_e4m3fn, as torch's
  * `tensor.to(torch.float8_e4m3fn)`: round to nearest even, |x| rounding past
  * 448, +-inf and NaN -> NaN (0x7F | sign).  Replaces the FP8 path of

@@ -606,6 +606,26 @@ int lrq_act_qdq(const void* in, int in_dtype, int64_t rows, int64_t cols, int64_
                    "kernel launch");
 }
 
+int lrq_fp8_linear(const void* x, int x_dtype, int64_t rows, int64_t k, int64_t ld, const uint8_t* codes,
+                   const void* scales, int64_t n, const void* bias, int bias_dtype, void* out, lrq_stream_t stream) {
+  g_err.clear();
+  if (x_dtype != lrq::kBF16 && x_dtype != lrq::kF16) return fail(LRQ_ERR_ARG, "bad activation dtype %d", x_dtype);
+  if (bias && !valid_dtype(bias_dtype)) return fail(LRQ_ERR_ARG, "bad bias dtype %d", bias_dtype);
+  if (rows < 0 || n < 0 || k < 0 || k % lrq::kLinBlock != 0)
+    return fail(LRQ_ERR_ARG, "k (%lld) must be a multiple of 128", (long long)k);
+  if (rows > lrq::kLinRowsMax || n > INT32_MAX || k > lrq::kLinPitchMax || ld > lrq::kLinPitchMax)
+    return fail(LRQ_ERR_ARG, "linear of %lld x %lld x %lld (pitch %lld) is too large", (long long)rows, (long long)n,
+                (long long)k, (long long)ld);
+  if (rows == 0 || n == 0) return 0;
+  if (k == 0 || ld < k) return fail(LRQ_ERR_ARG, "ld < k, or k is 0");
+  if (!x || !codes || !scales || !out) return fail(LRQ_ERR_ARG, "null pointer");
+  if (!aligned(x, 2) || !aligned(codes, 16) || !aligned(scales, 2) || !aligned(out, 16) ||
+      (bias && !aligned(bias, (uintptr_t)esize(bias_dtype))))
+    return fail(LRQ_ERR_ALIGN, "x, scales and bias must be element-aligned, codes and out 16-byte aligned");
+  const lrq::LinearArgs a{x, codes, static_cast<const uint16_t*>(scales), bias, out, ld, rows, n, k, bias_dtype};
+  return check_hip(lrq::launch_linear(a, x_dtype, (hipStream_t)stream), "kernel launch");
+}
+
 int lrq_cast_e4m3(const void* in, int in_dtype, int64_t n, uint8_t* out, lrq_stream_t stream) {
   g_err.clear();
   lrq_tensor t{in, out, nullptr, 1, 1, n, n, n};

@@ -235,6 +235,23 @@ int64_t act_grid(int dtype, int64_t rows, int64_t cols, int64_t blk);
 hipError_t launch_act(const void* in, int dtype, int64_t rows, int64_t cols, int64_t ld, int64_t blk,
                       float* out, int pow2, hipStream_t stream);
 
+// The FP8 rollout linear: y [m, n] = x [m, k] (row pitch ldx) times the
+// transpose of the dequantized weight [n, k] (dense e4m3 codes, bf16 scales
+// [n, k / kLinBlock]), plus an optional bias [n]; y has x's 16-bit type.
+constexpr int64_t kLinBlock = 128;
+constexpr int64_t kLinRowsMax = 64;       // tokens that k_linear_rows takes
+constexpr int64_t kLinPitchMax = 1 << 24; // row pitches: 32-bit byte offsets within a tile of rows
+struct LinearArgs {
+  const void* x;
+  const uint8_t* codes;
+  const uint16_t* scales;
+  const void* bias;  // null: none
+  void* y;
+  int64_t ldx, m, n, k;
+  int bias_dtype;
+};
+hipError_t launch_linear(const LinearArgs& a, int dtype, hipStream_t stream);
+
 // Diagnostics: element encoders applied to raw inputs.
 hipError_t launch_diag_e4m3_bits(uint32_t start, int64_t n, uint8_t* out, hipStream_t stream);
 hipError_t launch_diag_bf16_bits(uint32_t start, int64_t n, uint16_t* out, hipStream_t stream);

@@ -48,6 +48,7 @@ SIGNATURES = {
     "lrq_mxfp8_quant": (_CI, [_VP, _CI, _I64, _I64, _I64, _VP, _VP, _VP]),
     "lrq_mxfp4_quant": (_CI, [_VP, _CI, _I64, _I64, _I64, _VP, _VP, _VP]),
     "lrq_act_qdq": (_CI, [_VP, _CI, _I64, _I64, _I64, _I64, _CU, _VP, _VP]),
+    "lrq_fp8_linear": (_CI, [_VP, _CI, _I64, _I64, _I64, _VP, _VP, _I64, _VP, _CI, _VP, _VP]),
     "lrq_cast_e4m3": (_CI, [_VP, _CI, _I64, _VP, _VP]),
     "lrq_mx_dequant": (_CI, [_CI, _VP, _VP, _I64, _I64, _VP, _CI, _VP]),
     "lrq_group_table_bytes": (_I64, [_CI, ctypes.POINTER(LrqTensor), _I64, _CI, _I64, _I64, _CU]),

@@ -18,7 +18,7 @@ from lumenrl_amd.quantization.ops import (
     quantize_mxfp4,
     quantize_mxfp8,
 )
-from lumenrl_amd.quantization.ops import act_qdq, fp8_block_dequant, fp8_block_quant
+from lumenrl_amd.quantization.ops import act_qdq, fp8_block_dequant, fp8_block_quant, fp8_linear
 from lumenrl_amd.quantization.weight_quantizer import WeightQuantizer, fp8_e4m3_max
 
 __all__ = [
@@ -39,6 +39,7 @@ __all__ = [
     "fp8_block_dequant",
     "fp8_block_quant",
     "fp8_e4m3_max",
+    "fp8_linear",
     "quantize_fp8_blockwise",
     "quantize_mxfp4",
     "quantize_mxfp8",

@@ -213,6 +213,51 @@ def act_qdq(x: Tensor, block: int = 128, *, pow2: bool = False,
     return out
 
 
+FP8_LINEAR_MAX_TOKENS = 64        # fp8_linear: tokens (rows of x) of one call
+FP8_LINEAR_MAX_PITCH = 1 << 24    # fp8_linear: K, and the row pitch the kernel reads x with
+
+
+def fp8_linear(x: Tensor, codes: Tensor, scales: Tensor, bias: Optional[Tensor] = None) -> Tensor:
+    """The FP8 rollout linear (fp8_rollout.py:53-78) in one launch, for up to
+    ``FP8_LINEAR_MAX_TOKENS`` tokens.
+
+    ``x`` [..., K] bf16 or fp16, ``codes`` [N, K] float8_e4m3fn with bf16
+    ``scales`` [N, K/128] (both contiguous), ``bias`` [N] bf16, fp16 or fp32 ->
+    [prod(...), N] in x's dtype: act_qdq(x) @ dequantized(codes).T + bias with
+    float32 sums.
+    """
+    _check_input(x, "fp8_linear")
+    n, k = codes.shape
+    last = x.shape[-1]
+    if last != k or tuple(scales.shape) != (n, k // 128):
+        raise ValueError(f"fp8_linear: x {tuple(x.shape)}, codes {tuple(codes.shape)} and scales "
+                         f"{tuple(scales.shape)} do not fit")
+    if (codes.dtype != torch.float8_e4m3fn or scales.dtype != torch.bfloat16 or not codes.is_contiguous()
+            or not scales.is_contiguous() or codes.device != x.device or scales.device != x.device):
+        raise ValueError("fp8_linear: codes must be contiguous float8_e4m3fn and scales contiguous bfloat16, "
+                         f"both on {x.device}")
+    if bias is not None and (tuple(bias.shape) != (n,) or bias.dtype not in _IN_DTYPES or bias.device != x.device
+                             or not bias.is_contiguous()):
+        raise ValueError(f"fp8_linear: bias must be a contiguous [{n}] tensor on {x.device}")
+    rows = x.numel() // last if last else 0
+    xm = x.reshape(rows, last)
+    if xm.stride(-1) != 1:  # as act_qdq: any row pitch and element alignment, but unit-stride rows
+        xm = xm.contiguous()
+    out = torch.empty((rows, n), dtype=x.dtype, device=x.device)
+    if out.numel() == 0:
+        return out
+    ld = xm.stride(0) if rows > 1 else last
+    if ld > FP8_LINEAR_MAX_PITCH:
+        xm, ld = xm.contiguous(), last
+    with _on(x.device):
+        rc = _lib.lib().lrq_fp8_linear(xm.data_ptr(), _IN_DTYPES[x.dtype], rows, k, ld, codes.data_ptr(),
+                                       scales.data_ptr(), n, bias.data_ptr() if bias is not None else None,
+                                       _IN_DTYPES[bias.dtype] if bias is not None else 0, out.data_ptr(),
+                                       _stream(x.device))
+    _lib.check(rc, "lrq_fp8_linear")
+    return out
+
+
 def cast_e4m3(x: Tensor) -> Tensor:
     """``x.to(torch.float8_e4m3fn)`` on the device, unscaled (weight_loader.py:19-43):
     round to nearest even; |x| rounding past 448, +-inf and NaN give NaN."""

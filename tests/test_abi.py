@@ -561,3 +561,20 @@ def test_group_limit_counts_the_wide_kernels_work_group_size(dtype, blk_c, threa
     assert L().lrq_group_units(buf.ctypes.data) == limit
     rc, _ = pack(limit + 1)
     assert rc == _lib.ERR_ARG and "too large" in _lib.last_error()
+
+
+def test_fp8_linear_arguments_are_checked_before_any_device_call():
+    fake = ctypes.c_void_p(0x10000)
+    odd = ctypes.c_void_p(0x10001)
+
+    def call(x=fake, dt=0, rows=4, k=256, ld=256, codes=fake, scales=fake, n=64, bias=None, bdt=0, out=fake):
+        return L().lrq_fp8_linear(x, dt, rows, k, ld, codes, scales, n, bias, bdt, out, None)
+
+    assert call(rows=0) == 0 and call(n=0) == 0
+    for bad in ({"dt": 2}, {"dt": 7}, {"k": 200}, {"k": 0}, {"ld": 255}, {"ld": 0}, {"rows": -1}, {"n": -1},
+                {"rows": 65}, {"n": 1 << 31}, {"k": (1 << 24) + 128, "ld": 1 << 25}, {"ld": (1 << 24) + 1},
+                {"x": None}, {"codes": None}, {"scales": None}, {"out": None}, {"bias": fake, "bdt": 3}):
+        assert call(**bad) == _lib.ERR_ARG, bad
+    for bad in ({"x": odd}, {"codes": ctypes.c_void_p(0x10008)}, {"scales": odd}, {"out": ctypes.c_void_p(0x10004)},
+                {"bias": odd}):
+        assert call(**bad) == _lib.ERR_ALIGN, bad

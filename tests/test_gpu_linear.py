@@ -1,0 +1,162 @@
+"""The one-launch FP8 rollout linear (``ops.fp8_linear``) against a float64
+product of the same codes, scales and activations, and the calls that
+``_FP8W8A8Linear`` must still hand to the library product."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+import torch.nn as nn
+
+from lumenrl_amd.quantization import FP8Config, WeightQuantizer, fp8_linear, ops
+from lumenrl_amd.quantization import fp8_rollout
+from lumenrl_amd.quantization.fp8_rollout import _FP8W8A8Linear
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def operands(m, n, k, dtype, seed=0):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    x = torch.randn(m, k, generator=g, device=DEV)
+    x[:, k // 3] *= 40.0
+    codes = torch.randint(0, 256, (n, k), generator=g, device=DEV, dtype=torch.uint8)
+    codes[(codes & 0x7F) == 0x7F] = 0x30  # every code but the NaNs
+    scales = (torch.rand(n, k // 128, generator=g, device=DEV) + 0.5) * 1e-4
+    return x.to(dtype), codes.view(torch.float8_e4m3fn), scales.to(torch.bfloat16)
+
+
+def wide(codes, scales):
+    n, k = codes.shape
+    return (codes.to(torch.float64).view(n, -1, 128) * scales.to(torch.float64)[..., None]).view(n, k)
+
+
+def check(y, x, codes, scales, bias=None):
+    """|y - exact| within the result's own rounding and the float32 sums' bound:
+    no sum is longer than 128 products, K/128 blocks and 16 waves or parts, each
+    rounding (or truncating) by at most 2^-23 of the terms' magnitude; x_dq moves
+    a term by at most 2^-23 of itself."""
+    k = x.shape[-1]
+    w = wide(codes, scales)
+    xd = x.double().reshape(-1, k)
+    want, size = xd @ w.T, xd.abs() @ w.abs().T
+    if bias is not None:
+        want, size = want + bias.double(), size + bias.double().abs()
+    half_ulp = 2.0 ** -9 if y.dtype == torch.bfloat16 else 2.0 ** -12
+    bound = 2 * half_ulp * want.abs() + (128 + k // 128 + 20) * 2.0 ** -23 * size + 2.0 ** -24
+    off = (y.double() - want).abs()
+    assert bool((off <= bound).all()), float((off / bound).max())
+
+
+# tokens at the edges of the 16-row groups; weight rows at the edges of 16 to 64
+# row tiles and where the tile's shape changes; K of fewer blocks than waves,
+# an odd number of blocks and several per wave
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m", [1, 2, 16, 17, 33, 48, 49, 64])
+@pytest.mark.parametrize("n,k", [(1, 128), (15, 384), (17, 1152), (1000, 1024), (4099, 256), (12288, 256), (8200, 640)])
+def test_linear_vs_float64(dtype, m, n, k):
+    x, codes, scales = operands(m, n, k, dtype, seed=m * 7 + n)
+    y = fp8_linear(x, codes, scales)
+    assert y.dtype == dtype and y.shape == (m, n)
+    check(y, x, codes, scales)
+
+
+@pytest.mark.parametrize("bias_dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_linear_bias_strides_and_alignment(bias_dtype):
+    n, k = 264, 512
+    big, codes, scales = operands(40, n, 1600, torch.bfloat16, seed=3)
+    codes, scales = codes[:, :k].contiguous(), scales[:, :4].contiguous()
+    bias = torch.randn(n, device=DEV).to(bias_dtype)
+    for x in (big[:, :k], big[1:20, 3:3 + k], big[:, :2 * k:2], big[None, :6, :k].expand(1, 6, k), big[5, 7:7 + k]):
+        y = fp8_linear(x, codes, scales, bias)
+        check(y, x, codes, scales, bias)
+    with pytest.raises(ValueError):  # rows that share memory are refused, as by act_qdq
+        fp8_linear(big[:1, :k].expand(3, k), codes, scales)
+    with pytest.raises(ValueError):
+        fp8_linear(big[:, :k], codes[:, :384], scales)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_linear_non_finite_and_extreme_values(dtype):
+    n, k = 272, 512
+    x, codes, scales = operands(20, n, k, dtype, seed=9)
+    x[3, 100], x[4, 200], x[5, 300] = float("inf"), float("nan"), float("-inf")
+    x[6], x[7] = 0.0, torch.finfo(dtype).max / 2
+    x[8] = x[8].sign() * torch.finfo(dtype).tiny * 4
+    y = fp8_linear(x, codes, scales)
+    keep = [r for r in range(20) if r not in (3, 4, 5, 7)]
+    assert bool(y[3:6].isnan().all())  # s is inf or NaN: the whole block, so the whole row, is NaN
+    assert bool((y[6] == 0).all())
+    check(y[keep], x[keep], codes, scales)
+    # finite operands never overflow on the way: only where the result does
+    want = x[7].double() @ wide(codes, scales).T
+    fits = want.abs() < torch.finfo(dtype).max * 0.99
+    check(y[7:8][:, fits], x[7:8], codes[fits], scales[fits])
+    over = want.abs() > torch.finfo(dtype).max * 1.01
+    assert bool((y[7][over] == torch.where(want[over] > 0, float("inf"), float("-inf")).to(dtype)).all())
+    bad = codes.view(torch.uint8).clone()
+    bad[5, 40] = 0x7F  # a NaN code: that row of the weight, for every token
+    y = fp8_linear(x[8:12], bad.view(torch.float8_e4m3fn), scales)
+    assert bool(y[:, 5].isnan().all()) and not bool(y[:, 6:].isnan().any())
+
+
+def module(out, cols, dtype, bias=True, blk=128):
+    lin = nn.Linear(cols, out, bias=bias).to(DEV, dtype)
+    cfg = FP8Config(precision="fp8")
+    return _FP8W8A8Linear(lin, WeightQuantizer(cfg), cfg, blk)
+
+
+def test_module_routes(monkeypatch):
+    """The one-launch path where it applies; F.linear where autocast, the bias's
+    gradient, another block, type or device need it, with the results it gives."""
+    calls = []
+    real = ops.fp8_linear
+    monkeypatch.setattr(ops, "fp8_linear", lambda *a: calls.append(1) or real(*a))
+    torch.manual_seed(1)
+    mod, x = module(1024, 512, torch.bfloat16), torch.randn(2, 9, 512, device=DEV, dtype=torch.bfloat16)
+
+    def taken(m, v):
+        calls.clear()
+        y = m(v)
+        return y, bool(calls)
+
+    y_grad, fused = taken(mod, x)  # the bias wants a gradient
+    assert not fused and y_grad.requires_grad
+    with torch.no_grad():
+        y, fused = taken(mod, x)
+        assert fused and y.shape == (18, 1024) and y.dtype == torch.bfloat16
+        check(y, x, mod.weight_fp8, mod.weight_scale, mod.bias)
+        monkeypatch.setattr(fp8_rollout, "_ONE_LAUNCH_MIN_WEIGHT", 1 << 30)
+        y_lib, fused = taken(mod, x)
+        monkeypatch.setattr(fp8_rollout, "_ONE_LAUNCH_MIN_WEIGHT", 1 << 18)
+        # the same sums in another order: one unit of the last place where they round apart
+        assert not fused
+        assert bool(((y.double() - y_lib.double()).abs() <= 2.0 ** -7 * y_lib.double().abs() + 1e-5).all())
+        with torch.autocast("cuda", torch.bfloat16):
+            assert not taken(mod, x)[1]
+        assert not taken(mod, x.float())[1] and not taken(mod, x.double())[1] and not taken(mod, x.cpu())[1]
+        assert not taken(mod, x[:0])[1]
+        assert not taken(module(1024, 384, torch.bfloat16, blk=96), x[..., :384])[1]
+        assert not taken(module(384, 512, torch.bfloat16), x)[1]  # a small weight
+        with pytest.raises(RuntimeError):  # F.linear's own error for a width that is not the weight's
+            mod(x[..., :256])
+        half = module(1024, 512, torch.float16, bias=False)
+        y, fused = taken(half, x[0, 0].half())
+        assert fused and y.shape == (1, 1024)
+        check(y, x[0, :1].half(), half.weight_fp8, half.weight_scale)
+
+
+def test_linear_in_a_graph():
+    """Captured and replayed with new inputs and eager work between the replays."""
+    x, codes, scales = operands(8, 1024, 512, torch.bfloat16)
+    fp8_linear(x, codes, scales)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = fp8_linear(x, codes, scales)
+    for seed in range(3):
+        x.copy_(operands(8, 1024, 512, torch.bfloat16, seed=seed + 20)[0])
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(y.view(torch.int16).cpu().numpy(), fp8_linear(x, codes, scales).view(torch.int16).cpu().numpy())
