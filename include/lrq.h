@@ -150,7 +150,7 @@ int lrq_act_qdq(const void* in, int in_dtype, int64_t rows, int64_t cols, int64_
                 unsigned flags, float* out, lrq_stream_t stream);
 
 /*
- * The FP8 rollout linear for few tokens in one launch:
+ * The FP8 rollout linear in one launch:
  *   out[m, n] = x_dq[m, k] . w_dq[n, k]^T + bias[n]
  * with x_dq as lrq_act_qdq (blk 128) and w_dq as lrq_fp8_block_dequant (1 x 128
  * blocks) give them, float32 sums and a result in x's type.  Replaces
@@ -161,7 +161,8 @@ int lrq_act_qdq(const void* in, int in_dtype, int64_t rows, int64_t cols, int64_
  *   codes  : [n, k] e4m3 bytes, dense;  scales : [n, k/128] bf16, dense;
  *   bias   : [n] of bias_dtype (bf16, fp16 or fp32), or null;
  *   out    : [rows, n] of x's type, dense, 16-byte aligned.
- * rows <= 64; k a multiple of 128; k and ld at most 2^24.
+ * k a multiple of 128; k and ld at most 2^24; rows and n below 2^31 and rows * n
+ * below 2^37.
  */
 int lrq_fp8_linear(const void* x, int x_dtype, int64_t rows, int64_t k, int64_t ld,
                    const uint8_t* codes, const void* scales, int64_t n, const void* bias,

@@ -239,7 +239,6 @@ hipError_t launch_act(const void* in, int dtype, int64_t rows, int64_t cols, int
 // transpose of the dequantized weight [n, k] (dense e4m3 codes, bf16 scales
 // [n, k / kLinBlock]), plus an optional bias [n]; y has x's 16-bit type.
 constexpr int64_t kLinBlock = 128;
-constexpr int64_t kLinRowsMax = 64;       // tokens that k_linear_rows takes
 constexpr int64_t kLinPitchMax = 1 << 24; // row pitches: 32-bit byte offsets within a tile of rows
 struct LinearArgs {
   const void* x;
@@ -250,6 +249,7 @@ struct LinearArgs {
   int64_t ldx, m, n, k;
   int bias_dtype;
 };
+int64_t linear_grid(int64_t m, int64_t n);  // work-groups at most, but for few tokens
 hipError_t launch_linear(const LinearArgs& a, int dtype, hipStream_t stream);
 
 // Diagnostics: element encoders applied to raw inputs.

@@ -289,24 +289,261 @@ __global__ __launch_bounds__(64 * KW) void k_linear_rows(LinearArgs a) {
   }
 }
 
-// Tile of y per work-group, in units of 16 tokens and 16 weight rows.  Its
-// cost is the bytes that its CU moves through the vector cache and LDS, 2 mt +
-// nt (x has two bytes an element), times the rounds of work-groups that the 256
-// CUs take; the shape with the least cost is within 5 % of the fastest that a
-// sweep over all of them found at 1 to 64 tokens and weights of [1024 to 12288,
-// 4096 to 12288].
-struct RowsShape {
-  int mt, nt;
-};
-static RowsShape rows_shape(int64_t m, int64_t n) {
-  RowsShape best{1, 1};
-  int64_t least = INT64_MAX;
-  for (int mt = 1; mt <= 4 && 16 * (mt - 1) < m; ++mt)
-    for (int nt = 1; nt <= 4; ++nt) {
-      const int64_t wgs = ((n + 16 * nt - 1) / (16 * nt)) * ((m + 16 * mt - 1) / (16 * mt));
-      const int64_t cost = ((wgs + 255) / 256) * (2 * mt + nt);
-      if (cost < least) least = cost, best = {mt, nt};
+// ---------------------------------------------------------------------------
+// Many tokens (prefill): bound by the matrix cores
+// ---------------------------------------------------------------------------
+// A work-group of WM x WN waves makes a tile of y of 16 FM WM tokens and 16 FN
+// WN weight rows; each wave its (16 FM) x (16 FN) of it.  Blocks of 128 k go
+// through two LDS buffers: x as it is and the weight as e4m3 bytes, which each
+// wave converts for itself (half the LDS traffic of 16-bit weights).  A wave
+// keeps the block of its own x rows in registers and takes the weight 16 rows
+// at a time: 4 FM matrix instructions, whose float32 sums the block's scale
+// then multiplies into the accumulators.  That multiplication runs one step
+// behind, between the next step's matrix instructions, and so do the
+// conversions, the moves of the next block into LDS and the loads of the one
+// after: 3 vector instructions fit beside each matrix instruction.
+//
+// 8 x 4 x (1 x 4): 128 x 256 tiles, one work-group of 4 waves on a CU.  A wave
+// of 128 x 64 reads 40 KiB of LDS a block for 128 matrix instructions, where 64
+// x 64 (8 waves, the same tile) would read 48 and saturate LDS; 64 x 128 reads
+// less but converts every code twice (2 % slower).  8192 tokens x [12288, 4096]
+// take 0.90 ms (919 TFLOP/s), 5.6 ms before by way of float32 operands and a
+// float32 library product (147 TFLOP/s).
+// 2 x 4 x (2 x 2): 64 x 128 tiles, two work-groups on a CU, for grids that would
+// leave CUs idle with the larger tile: 512 tokens x [4096, 4096] 34 us (46 to 76
+// on larger tiles).
+//
+// The compiler keeps the matrix instructions' results in vector registers
+// (-amdgpu-mfma-vgpr-form): in accumulation registers, its own choice here,
+// every result needed a move before the scale could multiply it (15 % slower).
+// The tile of work-group `wg`.  Work-groups go to the 8 XCDs in turn; each XCD
+// takes one run of the tiles, walked 8 tile rows at a time, so that the rows of
+// x and of the weight that its work-groups read together stay in its L2.
+__device__ __forceinline__ void linear_tile(int wg, int tiles_m, int tiles_n, int& tm, int& tn) {
+  const int tiles = tiles_m * tiles_n, per = tiles >> 3;
+  const int t = wg < 8 * per ? (wg & 7) * per + (wg >> 3) : wg;
+  const int group = 8 * tiles_n, first = t / group * 8;
+  const int rows = tiles_m - first < 8 ? tiles_m - first : 8;
+  tm = first + (t % group) % rows;
+  tn = (t % group) / rows;
+}
+
+// Barrier of the work-group for its LDS accesses only: loads from memory stay
+// in flight across it.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+template <int DT, int FM, int FN, int WM, int WN>
+__global__ __launch_bounds__(64 * WM * WN, 1) void k_linear_tiles(LinearArgs a, int tiles_m, int tiles_n) {
+  constexpr int T = 64 * WM * WN, BM = 16 * FM * WM, BN = 16 * FN * WN;
+  constexpr int PA = BM * 16 / T, PB = BN * 8 / T;   // 16-byte pieces a thread moves per K block
+  constexpr int kA = BM * 256, kB = BN * 128, kBuf = kA + kB + BN * 4;
+  static_assert(BN <= T && PA * T == BM * 16 && PB * T == BN * 8, "");
+  __shared__ __attribute__((aligned(16))) uint8_t lds[2 * kBuf];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 15, g = lane >> 4;
+  int tm, tn;
+  linear_tile(blockIdx.x, tiles_m, tiles_n, tm, tn);
+  const int m0 = tm * BM, n0 = tn * BN;
+  const int n_last = (int)a.n - 1 - n0, m_last = (int)a.m - 1 - m0;
+  const int kb_n = (int)(a.k / kLinBlock);
+  const uint8_t* const w0 = a.codes + (int64_t)n0 * a.k;
+  const uint16_t* const s0 = a.scales + (int64_t)n0 * kb_n;
+  const uint8_t* const x0 = static_cast<const uint8_t*>(a.x) + 2 * (m0 * a.ldx);
+  uint32_t xo[PA], wo[PB];
+#pragma unroll
+  for (int p = 0; p < PA; ++p) {
+    const int r = (T / 16) * p + (tid >> 4);
+    xo[p] = (uint32_t)(r < m_last ? r : m_last) * (uint32_t)(2 * a.ldx) + 16 * (tid & 15);
+  }
+#pragma unroll
+  for (int p = 0; p < PB; ++p) {
+    const int r = (T / 8) * p + (tid >> 3);
+    wo[p] = (uint32_t)(r < n_last ? r : n_last) * (uint32_t)a.k + 16 * (tid & 7);
+  }
+  const int sr = tid < BN ? tid : BN - 1;  // the scale this thread moves
+  const uint32_t so = (uint32_t)(sr < n_last ? sr : n_last) * (uint32_t)kb_n;
+  v4u gx[PA], gw[PB];
+  uint32_t gs;
+  // The moves of a block are spread over the tiles j = 0 .. FN - 2 of the block
+  // before: stores into LDS in the first half, loads in the second.
+  constexpr int HP = (FN - 1) / 2, HF = FN - 1 - HP;
+  auto fetch = [&](int kb, int j) {
+    kb = kb < kb_n ? kb : kb_n - 1;
+    const uint8_t* const xb = x0 + 2 * (kb * kLinBlock);
+    const uint8_t* const wb = w0 + kb * kLinBlock;
+#pragma unroll
+    for (int p = 0; p < PA; ++p)
+      if (j == HP + p * HF / PA) gx[p] = load_x16(xb + xo[p]);
+#pragma unroll
+    for (int p = 0; p < PB; ++p)
+      if (j == HP + p * HF / PB) gw[p] = load_x16(wb + wo[p]);
+    if (j == HP) gs = gld<uint16_t>(s0 + kb + so);
+  };
+  auto put = [&](uint8_t* buf, int j) {
+#pragma unroll
+    for (int p = 0; p < PA; ++p) {
+      const int r = (T / 16) * p + (tid >> 4);
+      if (j == p * HP / PA) *reinterpret_cast<v4u*>(buf + 256 * r + 16 * ((tid & 15) ^ (r & 15))) = gx[p];
     }
+#pragma unroll
+    for (int p = 0; p < PB; ++p) {
+      const int r = (T / 8) * p + (tid >> 3);
+      if (j == p * HP / PB) *reinterpret_cast<v4u*>(buf + kA + 128 * r + 16 * ((tid & 7) ^ ((r >> 1) & 7))) = gw[p];
+    }
+    if (j == 0 && (BN == T || tid < BN)) *reinterpret_cast<uint32_t*>(buf + kA + kB + 4 * tid) = gs << 16;
+  };
+  const int wm = (wave / WN) * 16 * FM, wn = (wave % WN) * 16 * FN;
+  v4u xa[FM][4], wr[2];
+  auto read_x = [&](const uint8_t* buf, int q) {
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+        xa[i][q] = *reinterpret_cast<const v4u*>(buf + 256 * (wm + 16 * i + c) + 16 * ((2 * (g + 4 * (q >> 1)) + (q & 1)) ^ c));
+  };
+  auto read_w = [&](const uint8_t* buf, int j) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      wr[h] = *reinterpret_cast<const v4u*>(buf + kA + 128 * (wn + 16 * j + c) + 16 * ((g + 4 * h) ^ (c >> 1)));
+  };
+  f32x4 acc[FM][FN], p[FM], pp[FM];
+  float sp = 0.0f;
+#pragma unroll
+  for (int i = 0; i < FM; ++i) {
+    pp[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int j = 0; j < FN; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  }
+#pragma unroll
+  for (int j = 0; j + 1 < FN; ++j) fetch(0, j);
+#pragma unroll
+  for (int j = 0; j + 1 < FN; ++j) put(lds, j);
+#pragma unroll
+  for (int j = 0; j + 1 < FN; ++j) fetch(1, j);
+  lds_barrier();
+#pragma unroll
+  for (int q = 0; q < 4; ++q) read_x(lds, q);
+  read_w(lds, 0);
+  for (int kb = 0; kb < kb_n; ++kb) {
+    const uint8_t* const cur = lds + (kb & 1) * kBuf;
+    uint8_t* const nxt = lds + ((kb + 1) & 1) * kBuf;
+    float sc[FN];
+#pragma unroll
+    for (int j = 0; j < FN; ++j) sc[j] = *reinterpret_cast<const float*>(cur + kA + kB + 4 * (wn + 16 * j + c));
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+      const v4u w[2] = {wr[0], wr[1]};
+      if (j + 1 < FN) {
+        read_w(cur, j + 1);
+        // the next block goes into LDS during the first tiles, the one after it
+        // is fetched during the next
+        put(nxt, j);
+        fetch(kb + 2, j);
+      } else {
+        lds_barrier();  // every read of `cur` is done and `nxt` is whole
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const v4u b = (q & 1) ? codes_to_x16<DT>(w[q >> 1].z, w[q >> 1].w) : codes_to_x16<DT>(w[q >> 1].x, w[q >> 1].y);
+#pragma unroll
+        for (int i = 0; i < FM; ++i) p[i] = mfma16<DT>(xa[i][q], b, q ? p[i] : f32x4{0.0f, 0.0f, 0.0f, 0.0f});
+        if (j + 1 == FN) {
+          if (q == 0) read_w(nxt, 0);
+          read_x(nxt, q);
+        }
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+          acc[i][(j + FN - 1) % FN][q] = __builtin_fmaf(pp[i][q], sp, acc[i][(j + FN - 1) % FN][q]);
+      }
+#pragma unroll
+      for (int i = 0; i < FM; ++i) pp[i] = p[i];
+      sp = sc[j];
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) acc[i][FN - 1][r] = __builtin_fmaf(pp[i][r], sp, acc[i][FN - 1][r]);
+  // The wave's part of y goes through its own piece of LDS (no block is read
+  // any more), so that rows leave in 16-byte stores.
+  constexpr int ROWS = 16 * FM, COLS = 16 * FN, PITCH = 2 * COLS + 16, PIECES = COLS / 8;
+  static_assert(WM * WN * ROWS * PITCH <= 2 * kBuf, "the tile of y fits where the blocks were");
+  uint8_t* const out = lds + wave * (ROWS * PITCH);
+  lds_barrier();
+  bool inf = false;
+#pragma unroll
+  for (int j = 0; j < FN; ++j) {
+    const int n = wn + 16 * j + c;
+    const float bias = a.bias != nullptr && n <= n_last ? linear_bias(a, n0 + n) : 0.0f;
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float sum = acc[i][j][r] * (1.0f / kCodeUnit<DT>);
+        inf |= (f2u(sum) & 0x7FFFFFFFu) == 0x7F800000u;
+        *reinterpret_cast<uint16_t*>(out + (16 * i + 4 * g + r) * PITCH + 2 * (16 * j + c)) = linear_bits<DT>(sum + bias);
+      }
+  }
+  wave_lds_fence();
+  if (__any(inf)) {  // rare: see linear_out
+    for (int e = lane; e < ROWS * COLS; e += 64) {
+      const int m = e / COLS, n = e % COLS;
+      uint16_t* const v = reinterpret_cast<uint16_t*>(out + m * PITCH + 2 * n);
+      if (wm + m <= m_last && wn + n <= n_last && (*v & 0x7FFFu) == (DT == kBF16 ? 0x7F80u : 0x7C00u) &&
+          linear_is_nan<DT>(a, m0 + wm + m, n0 + wn + n))
+        *v = DT == kBF16 ? 0x7FC0u : 0x7E00u;
+    }
+    wave_lds_fence();
+  }
+  const bool whole = a.n % 8 == 0;  // pieces of 8 columns are all in or all out, and 16-byte aligned
+#pragma unroll 4
+  for (int e = lane; e < ROWS * PIECES; e += 64) {
+    const int m = e / PIECES, q = e % PIECES, n = wn + 8 * q;
+    if (wm + m > m_last || n > n_last) continue;
+    uint16_t* const dst = static_cast<uint16_t*>(a.y) + (int64_t)(m0 + wm + m) * a.n + n0 + n;
+    const uint8_t* const src = out + m * PITCH + 16 * q;
+    if (whole) {
+      gst<v4u>(dst, *reinterpret_cast<const v4u*>(src));
+    } else {
+      for (int k = 0; k < 8 && n + k <= n_last; ++k) gst<uint16_t>(dst + k, reinterpret_cast<const uint16_t*>(src)[k]);
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Which kernel
+// ---------------------------------------------------------------------------
+// The shape with the least modelled time per 128-element K block, in ns:
+//   * k_linear_rows: the bytes that a CU moves through its vector cache and LDS,
+//     2 mt + nt units (x has two bytes an element), 55 ns each, times the rounds
+//     of work-groups that the 256 CUs take;
+//   * k_linear_tiles: 2340 ns a round of 128 x 256 tiles, one on a CU; of 64 x 128
+//     tiles 1060 ns where each has a CU to itself, else 1470 ns a round of two on
+//     each.
+// From sweeps over all shapes at 1 to 8192 tokens and weights of [1000 to 12288,
+// 1024 to 12288]; the shape it takes is within 5 % of the fastest up to 64 tokens
+// and 8 % beyond.
+struct LinearShape {
+  int tiles;   // 0: k_linear_rows, 1: 128 x 256 tiles, 2: 64 x 128 tiles
+  int mt, nt;  // k_linear_rows: tokens and weight rows per work-group, in 16s
+};
+static int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
+static LinearShape linear_shape(int64_t m, int64_t n) {
+  const int64_t large = ceil_div(m, 128) * ceil_div(n, 256), small = ceil_div(m, 64) * ceil_div(n, 128);
+  LinearShape best{1, 0, 0};
+  int64_t least = 2340 * ceil_div(large, 256);
+  const int64_t cost = small <= 256 ? 1060 : 1470 * ceil_div(small, 512);
+  if (cost < least) least = cost, best = {2, 0, 0};
+  for (int mt = 1; mt <= 4 && 16 * (mt - 1) < m; ++mt) {
+    if (ceil_div(m, 16 * mt) > 65535) continue;  // the grid's second dimension
+    for (int nt = 1; nt <= 4; ++nt) {
+      const int64_t rows = 55 * (2 * mt + nt) * ceil_div(ceil_div(n, 16 * nt) * ceil_div(m, 16 * mt), 256);
+      if (rows < least) least = rows, best = {0, mt, nt};
+    }
+  }
   return best;
 }
 
@@ -314,7 +551,7 @@ template <int DT, int MT, int NT>
 static void launch_rows(const LinearArgs& a, hipStream_t stream) {
   // 8 waves where their LDS (2 KiB per 16 weight rows and 4 per 16 tokens each) fits the CU's 160 KiB
   constexpr int KW = 8 * (2 * NT + 4 * MT) <= 144 ? 8 : 4;
-  const dim3 grid((unsigned)((a.n + 16 * NT - 1) / (16 * NT)), (unsigned)((a.m + 16 * MT - 1) / (16 * MT)));
+  const dim3 grid((unsigned)ceil_div(a.n, 16 * NT), (unsigned)ceil_div(a.m, 16 * MT));
   hipLaunchKernelGGL((k_linear_rows<DT, MT, NT, KW, 1>), grid, dim3(64 * KW), 0, stream, a);
 }
 template <int DT, int MT>
@@ -326,9 +563,17 @@ static void launch_rows_nt(const LinearArgs& a, int nt, hipStream_t stream) {
     default: launch_rows<DT, MT, 4>(a, stream); break;
   }
 }
+template <int DT, int FM, int FN, int WM, int WN>
+static void launch_tiles(const LinearArgs& a, hipStream_t stream) {
+  const int tiles_m = (int)ceil_div(a.m, 16 * FM * WM), tiles_n = (int)ceil_div(a.n, 16 * FN * WN);
+  hipLaunchKernelGGL((k_linear_tiles<DT, FM, FN, WM, WN>), dim3((unsigned)(tiles_m * tiles_n)), dim3(64 * WM * WN), 0,
+                     stream, a, tiles_m, tiles_n);
+}
 template <int DT>
-static void launch_rows_shape(const LinearArgs& a, hipStream_t stream) {
-  const RowsShape s = rows_shape(a.m, a.n);
+static void launch_linear_dt(const LinearArgs& a, hipStream_t stream) {
+  const LinearShape s = linear_shape(a.m, a.n);
+  if (s.tiles == 1) return launch_tiles<DT, 8, 4, 1, 4>(a, stream);
+  if (s.tiles == 2) return launch_tiles<DT, 2, 4, 2, 2>(a, stream);
   switch (s.mt) {
     case 1: launch_rows_nt<DT, 1>(a, s.nt, stream); break;
     case 2: launch_rows_nt<DT, 2>(a, s.nt, stream); break;
@@ -337,9 +582,12 @@ static void launch_rows_shape(const LinearArgs& a, hipStream_t stream) {
   }
 }
 
+// Work-groups of the smallest tile any shape has: the host refuses grids past 2^24.
+int64_t linear_grid(int64_t m, int64_t n) { return ceil_div(m, 64) * ceil_div(n, 128); }
+
 hipError_t launch_linear(const LinearArgs& a, int dtype, hipStream_t stream) {
-  if (dtype == kBF16) launch_rows_shape<kBF16>(a, stream);
-  else launch_rows_shape<kF16>(a, stream);
+  if (dtype == kBF16) launch_linear_dt<kBF16>(a, stream);
+  else launch_linear_dt<kF16>(a, stream);
   return hipGetLastError();
 }
 

@@ -213,13 +213,12 @@ def act_qdq(x: Tensor, block: int = 128, *, pow2: bool = False,
     return out
 
 
-FP8_LINEAR_MAX_TOKENS = 64        # fp8_linear: tokens (rows of x) of one call
-FP8_LINEAR_MAX_PITCH = 1 << 24    # fp8_linear: K, and the row pitch the kernel reads x with
+FP8_LINEAR_MAX_PITCH = 1 << 24  # fp8_linear: K, and the row pitch the kernels read x with
+FP8_LINEAR_MAX_CELLS = 1 << 36  # fp8_linear: tokens * out_features
 
 
 def fp8_linear(x: Tensor, codes: Tensor, scales: Tensor, bias: Optional[Tensor] = None) -> Tensor:
-    """The FP8 rollout linear (fp8_rollout.py:53-78) in one launch, for up to
-    ``FP8_LINEAR_MAX_TOKENS`` tokens.
+    """The FP8 rollout linear (fp8_rollout.py:53-78) in one launch.
 
     ``x`` [..., K] bf16 or fp16, ``codes`` [N, K] float8_e4m3fn with bf16
     ``scales`` [N, K/128] (both contiguous), ``bias`` [N] bf16, fp16 or fp32 ->

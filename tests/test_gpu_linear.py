@@ -62,13 +62,27 @@ def test_linear_vs_float64(dtype, m, n, k):
     check(y, x, codes, scales)
 
 
+# many tokens: 64 x 128 and 128 x 256 tiles with whole and cut last rows and
+# columns (also widths that 8 does not divide, stored one by one), one block of K,
+# an odd number and an even one; grids of one round and of several
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,n,k", [(65, 4096, 256), (129, 12289, 128), (200, 1003, 1024), (512, 4096, 128),
+                                   (500, 4090, 384), (700, 4097, 256), (1024, 7168, 128), (1030, 6999, 256),
+                                   (1025, 6992, 384), (2049, 4095, 640), (4100, 8192, 128)])
+def test_linear_many_tokens_vs_float64(dtype, m, n, k):
+    x, codes, scales = operands(m, n, k, dtype, seed=m + n)
+    bias = torch.randn(n, device=DEV) if m % 2 else None
+    check(fp8_linear(x, codes, scales, bias), x, codes, scales, bias)
+
+
 @pytest.mark.parametrize("bias_dtype", [torch.bfloat16, torch.float16, torch.float32])
 def test_linear_bias_strides_and_alignment(bias_dtype):
     n, k = 264, 512
     big, codes, scales = operands(40, n, 1600, torch.bfloat16, seed=3)
     codes, scales = codes[:, :k].contiguous(), scales[:, :4].contiguous()
     bias = torch.randn(n, device=DEV).to(bias_dtype)
-    for x in (big[:, :k], big[1:20, 3:3 + k], big[:, :2 * k:2], big[None, :6, :k].expand(1, 6, k), big[5, 7:7 + k]):
+    tall = torch.randn(1100, 2 * k + 5, device=DEV).to(torch.bfloat16)
+    for x in (tall[:, 3:3 + k], tall[:600, :2 * k:2], big[:, :k], big[1:20, 3:3 + k], big[:, :2 * k:2], big[None, :6, :k].expand(1, 6, k), big[5, 7:7 + k]):
         y = fp8_linear(x, codes, scales, bias)
         check(y, x, codes, scales, bias)
     with pytest.raises(ValueError):  # rows that share memory are refused, as by act_qdq
@@ -77,15 +91,16 @@ def test_linear_bias_strides_and_alignment(bias_dtype):
         fp8_linear(big[:, :k], codes[:, :384], scales)
 
 
+@pytest.mark.parametrize("m,n", [(20, 272), (500, 4096), (1030, 7000)])  # each kernel
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-def test_linear_non_finite_and_extreme_values(dtype):
-    n, k = 272, 512
-    x, codes, scales = operands(20, n, k, dtype, seed=9)
+def test_linear_non_finite_and_extreme_values(dtype, m, n):
+    k = 512
+    x, codes, scales = operands(m, n, k, dtype, seed=9)
     x[3, 100], x[4, 200], x[5, 300] = float("inf"), float("nan"), float("-inf")
     x[6], x[7] = 0.0, torch.finfo(dtype).max / 2
     x[8] = x[8].sign() * torch.finfo(dtype).tiny * 4
     y = fp8_linear(x, codes, scales)
-    keep = [r for r in range(20) if r not in (3, 4, 5, 7)]
+    keep = [r for r in range(m) if r not in (3, 4, 5, 7)]
     assert bool(y[3:6].isnan().all())  # s is inf or NaN: the whole block, so the whole row, is NaN
     assert bool((y[6] == 0).all())
     check(y[keep], x[keep], codes, scales)
