@@ -614,7 +614,7 @@ int lrq_fp8_linear(const void* x, int x_dtype, int64_t rows, int64_t k, int64_t 
   if (rows < 0 || n < 0 || k < 0 || k % lrq::kLinBlock != 0)
     return fail(LRQ_ERR_ARG, "k (%lld) must be a multiple of 128", (long long)k);
   if (rows > INT32_MAX || n > INT32_MAX || k > lrq::kLinPitchMax || ld > lrq::kLinPitchMax ||
-      lrq::linear_grid(rows, n) > (1 << 24) - 1)
+      lrq::linear_grid(rows, n) > (1 << 25))
     return fail(LRQ_ERR_ARG, "linear of %lld x %lld x %lld (pitch %lld) is too large", (long long)rows, (long long)n,
                 (long long)k, (long long)ld);
   if (rows == 0 || n == 0) return 0;

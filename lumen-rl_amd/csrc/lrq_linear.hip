@@ -128,20 +128,26 @@ __device__ __forceinline__ uint16_t linear_out(const LinearArgs& a, float sum, i
 // The weight's e4m3 bytes are all that has to move; dequantizing it to float32
 // for a library product wrote and read 8 times as many.  On an MI355X, one token
 // through a 4096 x 4096 weight takes 6.6 us (48 us a call before) and 48 tokens
-// through 12288 x 4096 17.9 us (105 us), where the weight's bytes alone take
+// through 12288 x 4096 17.2 us (105 us), where the weight's bytes alone take
 // 2.5 and 7.6 us: at few work-groups per CU the rest is latency, and from about
 // 32 tokens on x's passage through each CU's cache and LDS.
 //
 // A work-group of KW waves makes a (16 MT) x (16 NT) tile of y over the whole
-// of K: wave w takes the 128-element K blocks w, w + KW, ... of all its rows,
-// and the waves' sums meet in LDS at the end.  A matrix-core operand wants 16
+// of K: each wave takes a run of 128-element K blocks of all its rows, and the
+// waves' sums meet in LDS at the end.  A matrix-core operand wants 16
 // different rows in 16 neighbouring lanes, and loads in that order fetch one
 // cache line per lane; so each wave loads whole 128-byte runs of codes (8 lanes
-// a row) and whole 256-byte runs of x (16 lanes a row) into registers, DEPTH
-// blocks ahead, and turns them round through its own few KiB of LDS.  A row's
+// a row) and whole 256-byte runs of x (16 lanes a row) into registers, a block
+// ahead, and turns them round through its own few KiB of LDS.  A row's
 // 16-byte pieces are stored at (piece ^ row)-like places, which makes both the
 // writes and the reads free of bank conflicts, and no other wave touches them,
-// so no barrier is needed until the end.
+// so no barrier is needed until the end.  Measured and left: runs of blocks
+// taken in turns by the waves (up to 10 % slower at one token), loads two or
+// four blocks ahead (the same, or spilled registers), K split over work-groups
+// with a second launch for the sums (slower but for K = 12288 at 32 tokens).
+//
+// ONCE: one work-group reads each weight row, past the caches (5 % faster); with
+// more token groups than one the others find the row in L2 (up to 25 % faster).
 template <int NT, int MT>
 struct LinStage {
   v4u w[NT][2];  // codes: rows 8 i + lane / 8, 16-byte piece lane % 8
@@ -149,7 +155,7 @@ struct LinStage {
   v4u x[MT][4];  // x: rows 4 i + lane / 16, 16-byte piece lane % 16
 };
 
-template <int DT, int MT, int NT, int KW, int DEPTH>
+template <int DT, int MT, int NT, int KW, bool ONCE>
 __global__ __launch_bounds__(64 * KW) void k_linear_rows(LinearArgs a) {
   constexpr int COLS = 16 * NT, CELLS = 16 * MT * COLS;
   constexpr int kStageBytes = NT * 2048 + MT * 4096;
@@ -188,16 +194,16 @@ __global__ __launch_bounds__(64 * KW) void k_linear_rows(LinearArgs a) {
   // Every wave runs the same number of steps, so that no load hangs on a branch
   // and the waits between loads and uses stay counted: a step past K reads the
   // last block again and scales its sums with 0.
-  const int steps = ((kb_n + KW - 1) / KW + DEPTH - 1) / DEPTH * DEPTH;
+  const int steps = (kb_n + KW - 1) / KW;
   auto load = [&](LinStage<NT, MT>& st, int t) {
-    const int kt = wave + t * KW, kb = kt < kb_n ? kt : kb_n - 1;
+    const int kt = wave * steps + t, kb = kt < kb_n ? kt : kb_n - 1;
     const uint32_t keep = kt < kb_n ? 0xFFFFu : 0u;
     const uint8_t* const wb = w0 + kb * kLinBlock;
     const uint8_t* const xb = x0 + 2 * (kb * kLinBlock);
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
-      st.w[j][0] = load_nt(wb + wo[j][0]);
-      st.w[j][1] = load_nt(wb + wo[j][1]);
+      st.w[j][0] = ONCE ? load_nt(wb + wo[j][0]) : load_x16(wb + wo[j][0]);
+      st.w[j][1] = ONCE ? load_nt(wb + wo[j][1]) : load_x16(wb + wo[j][1]);
       st.s[j] = gld<uint16_t>(s0 + kb + so[j]) & keep;
     }
 #pragma unroll
@@ -253,23 +259,21 @@ __global__ __launch_bounds__(64 * KW) void k_linear_rows(LinearArgs a) {
       }
     }
   };
-  LinStage<NT, MT> st[DEPTH];
+  LinStage<NT, MT> st;
+  float sc[NT];
+  auto turn = [&] {
 #pragma unroll
-  for (int d = 0; d < DEPTH; ++d) load(st[d], d);
-  auto step = [&](int d, int next) {
-    float sc[NT];
-#pragma unroll
-    for (int j = 0; j < NT; ++j) sc[j] = u2f(st[d].s[j] << 16);
-    stash(st[d]);
-    if (next > 0) load(st[d], next);
-    multiply(sc);
+    for (int j = 0; j < NT; ++j) sc[j] = u2f(st.s[j] << 16);
+    stash(st);
   };
-  for (int t = DEPTH; t < steps; t += DEPTH) {
-#pragma unroll
-    for (int d = 0; d < DEPTH; ++d) step(d, t + d);
+  load(st, 0);
+  for (int t = 1; t < steps; ++t) {
+    turn();
+    load(st, t);
+    multiply(sc);
   }
-#pragma unroll
-  for (int d = 0; d < DEPTH; ++d) step(d, 0);
+  turn();
+  multiply(sc);
   __syncthreads();  // the waves' own LDS becomes the shared sums
   float* const red = reinterpret_cast<float*>(lds);
 #pragma unroll
@@ -303,15 +307,16 @@ __global__ __launch_bounds__(64 * KW) void k_linear_rows(LinearArgs a) {
 // conversions, the moves of the next block into LDS and the loads of the one
 // after: 3 vector instructions fit beside each matrix instruction.
 //
-// 8 x 4 x (1 x 4): 128 x 256 tiles, one work-group of 4 waves on a CU.  A wave
-// of 128 x 64 reads 40 KiB of LDS a block for 128 matrix instructions, where 64
-// x 64 (8 waves, the same tile) would read 48 and saturate LDS; 64 x 128 reads
-// less but converts every code twice (2 % slower).  8192 tokens x [12288, 4096]
-// take 0.90 ms (919 TFLOP/s), 5.6 ms before by way of float32 operands and a
-// float32 library product (147 TFLOP/s).
-// 2 x 4 x (2 x 2): 64 x 128 tiles, two work-groups on a CU, for grids that would
-// leave CUs idle with the larger tile: 512 tokens x [4096, 4096] 34 us (46 to 76
-// on larger tiles).
+// 4 x 4 x (2 x 4): 128 x 256 tiles, one work-group of 8 waves on a CU, two to a
+// SIMD, so that one's vector instructions and waits fall beside the other's
+// matrix instructions (4 waves of 128 x 64 each: 0.90 ms instead of 0.80).
+// 8192 tokens x [12288, 4096] take 0.80 ms (1035 TFLOP/s, matrix cores 47 % busy
+// at 1.9 GHz), 5.6 ms before by way of float32 operands and a float32 library
+// product (147 TFLOP/s).
+// The smaller tiles are for grids that would leave CUs idle with the large one:
+// each CU does less work per byte that passes its LDS, 28 us for 512 tokens x
+// [4096, 4096] in 64 x 128 tiles (59 in 128 x 256), 113 us for 1024 x [12288,
+// 4096] in 128 x 192 (125).
 //
 // The compiler keeps the matrix instructions' results in vector registers
 // (-amdgpu-mfma-vgpr-form): in accumulation registers, its own choice here,
@@ -517,31 +522,40 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void k_linear_tiles(LinearArgs a, 
 // Which kernel
 // ---------------------------------------------------------------------------
 // The shape with the least modelled time per 128-element K block, in ns:
-//   * k_linear_rows: the bytes that a CU moves through its vector cache and LDS,
-//     2 mt + nt units (x has two bytes an element), 55 ns each, times the rounds
-//     of work-groups that the 256 CUs take;
-//   * k_linear_tiles: 2340 ns a round of 128 x 256 tiles, one on a CU; of 64 x 128
-//     tiles 1060 ns where each has a CU to itself, else 1470 ns a round of two on
-//     each.
-// From sweeps over all shapes at 1 to 8192 tokens and weights of [1000 to 12288,
-// 1024 to 12288]; the shape it takes is within 5 % of the fastest up to 64 tokens
-// and 8 % beyond.
+//   * k_linear_rows: kLinearRows ns a round of 256 work-groups.  It grows with the
+//     bytes that a CU moves through its vector cache and LDS, 2 mt + nt units (x
+//     has two bytes an element); shapes past 8 waves' LDS do not pay any more;
+//   * k_linear_tiles: `each` ns a round of tiles, one on a CU, and `once` more;
+//     three 64 x 64 tiles fit a CU, 280 ns apiece and 457 once.
+// From sweeps over all shapes at 1 to 8192 tokens and weights of [500 to 12288,
+// 1024 to 12288], where the shape it takes is 1 % from the fastest in the mean.
+constexpr int kLinearRows[3][4] = {{136, 190, 315, 380}, {165, 280, 400, 465}, {290, 380, 485, INT32_MAX}};
+struct LinearTile {
+  int m, n, each, once;
+};
+constexpr LinearTile kLinearTiles[] = {
+    {128, 256, 2075, -200}, {128, 192, 1720, -80}, {128, 128, 1330, -100}, {64, 128, 800, 75}, {64, 64, 398, 0}};
+constexpr int kLinearTileKinds = sizeof(kLinearTiles) / sizeof(kLinearTiles[0]);
 struct LinearShape {
-  int tiles;   // 0: k_linear_rows, 1: 128 x 256 tiles, 2: 64 x 128 tiles
+  int tile;    // index into kLinearTiles, or -1: k_linear_rows
   int mt, nt;  // k_linear_rows: tokens and weight rows per work-group, in 16s
 };
 static int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 static LinearShape linear_shape(int64_t m, int64_t n) {
-  const int64_t large = ceil_div(m, 128) * ceil_div(n, 256), small = ceil_div(m, 64) * ceil_div(n, 128);
-  LinearShape best{1, 0, 0};
-  int64_t least = 2340 * ceil_div(large, 256);
-  const int64_t cost = small <= 256 ? 1060 : 1470 * ceil_div(small, 512);
-  if (cost < least) least = cost, best = {2, 0, 0};
-  for (int mt = 1; mt <= 4 && 16 * (mt - 1) < m; ++mt) {
+  LinearShape best{0, 0, 0};
+  int64_t least = INT64_MAX;
+  for (int i = 0; i < kLinearTileKinds; ++i) {
+    const LinearTile& t = kLinearTiles[i];
+    const int64_t rounds = ceil_div(ceil_div(m, t.m) * ceil_div(n, t.n), 256);
+    int64_t cost = t.each * rounds + t.once;
+    if (t.m == 64 && t.n == 64 && 280 * rounds + 457 > cost) cost = 280 * rounds + 457;
+    if (cost < least) least = cost, best = {i, 0, 0};
+  }
+  for (int mt = 1; mt <= 3 && 16 * (mt - 1) < m; ++mt) {
     if (ceil_div(m, 16 * mt) > 65535) continue;  // the grid's second dimension
-    for (int nt = 1; nt <= 4; ++nt) {
-      const int64_t rows = 55 * (2 * mt + nt) * ceil_div(ceil_div(n, 16 * nt) * ceil_div(m, 16 * mt), 256);
-      if (rows < least) least = rows, best = {0, mt, nt};
+    for (int nt = 1; nt <= (mt < 3 ? 4 : 3); ++nt) {
+      const int64_t cost = kLinearRows[mt - 1][nt - 1] * ceil_div(ceil_div(n, 16 * nt) * ceil_div(m, 16 * mt), 256);
+      if (cost < least) least = cost, best = {-1, mt, nt};
     }
   }
   return best;
@@ -549,18 +563,19 @@ static LinearShape linear_shape(int64_t m, int64_t n) {
 
 template <int DT, int MT, int NT>
 static void launch_rows(const LinearArgs& a, hipStream_t stream) {
-  // 8 waves where their LDS (2 KiB per 16 weight rows and 4 per 16 tokens each) fits the CU's 160 KiB
-  constexpr int KW = 8 * (2 * NT + 4 * MT) <= 144 ? 8 : 4;
-  const dim3 grid((unsigned)ceil_div(a.n, 16 * NT), (unsigned)ceil_div(a.m, 16 * MT));
-  hipLaunchKernelGGL((k_linear_rows<DT, MT, NT, KW, 1>), grid, dim3(64 * KW), 0, stream, a);
+  constexpr int KW = 8;  // their LDS, 2 KiB per 16 weight rows and 4 per 16 tokens each, fits the CU's 160 KiB
+  const dim3 grid((unsigned)ceil_div(a.n, 16 * NT), (unsigned)ceil_div(a.m, 16 * MT)), block(64 * KW);
+  if (grid.y == 1) hipLaunchKernelGGL((k_linear_rows<DT, MT, NT, KW, true>), grid, block, 0, stream, a);
+  else hipLaunchKernelGGL((k_linear_rows<DT, MT, NT, KW, false>), grid, block, 0, stream, a);
 }
 template <int DT, int MT>
 static void launch_rows_nt(const LinearArgs& a, int nt, hipStream_t stream) {
   switch (nt) {
-    case 1: launch_rows<DT, MT, 1>(a, stream); break;
-    case 2: launch_rows<DT, MT, 2>(a, stream); break;
-    case 3: launch_rows<DT, MT, 3>(a, stream); break;
-    default: launch_rows<DT, MT, 4>(a, stream); break;
+    case 1: return launch_rows<DT, MT, 1>(a, stream);
+    case 2: return launch_rows<DT, MT, 2>(a, stream);
+    case 3: return launch_rows<DT, MT, 3>(a, stream);
+    default:
+      if constexpr (MT < 3) launch_rows<DT, MT, 4>(a, stream);
   }
 }
 template <int DT, int FM, int FN, int WM, int WN>
@@ -570,24 +585,28 @@ static void launch_tiles(const LinearArgs& a, hipStream_t stream) {
                      stream, a, tiles_m, tiles_n);
 }
 template <int DT>
-static void launch_linear_dt(const LinearArgs& a, hipStream_t stream) {
-  const LinearShape s = linear_shape(a.m, a.n);
-  if (s.tiles == 1) return launch_tiles<DT, 8, 4, 1, 4>(a, stream);
-  if (s.tiles == 2) return launch_tiles<DT, 2, 4, 2, 2>(a, stream);
+static void launch_linear_dt(const LinearArgs& a, const LinearShape& s, hipStream_t stream) {
+  switch (s.tile) {
+    case 0: return launch_tiles<DT, 4, 4, 2, 4>(a, stream);
+    case 1: return launch_tiles<DT, 4, 3, 2, 4>(a, stream);
+    case 2: return launch_tiles<DT, 2, 2, 4, 4>(a, stream);
+    case 3: return launch_tiles<DT, 2, 2, 2, 4>(a, stream);
+    case 4: return launch_tiles<DT, 2, 2, 2, 2>(a, stream);
+  }
   switch (s.mt) {
-    case 1: launch_rows_nt<DT, 1>(a, s.nt, stream); break;
-    case 2: launch_rows_nt<DT, 2>(a, s.nt, stream); break;
-    case 3: launch_rows_nt<DT, 3>(a, s.nt, stream); break;
-    default: launch_rows_nt<DT, 4>(a, s.nt, stream); break;
+    case 1: return launch_rows_nt<DT, 1>(a, s.nt, stream);
+    case 2: return launch_rows_nt<DT, 2>(a, s.nt, stream);
+    default: return launch_rows_nt<DT, 3>(a, s.nt, stream);
   }
 }
 
-// Work-groups of the smallest tile any shape has: the host refuses grids past 2^24.
-int64_t linear_grid(int64_t m, int64_t n) { return ceil_div(m, 64) * ceil_div(n, 128); }
+// Work-groups of the smallest tile: the host refuses grids past 2^24 / 2.
+int64_t linear_grid(int64_t m, int64_t n) { return ceil_div(m, 64) * ceil_div(n, 64); }
 
 hipError_t launch_linear(const LinearArgs& a, int dtype, hipStream_t stream) {
-  if (dtype == kBF16) launch_linear_dt<kBF16>(a, stream);
-  else launch_linear_dt<kF16>(a, stream);
+  const LinearShape s = linear_shape(a.m, a.n);
+  if (dtype == kBF16) launch_linear_dt<kBF16>(a, s, stream);
+  else launch_linear_dt<kF16>(a, s, stream);
   return hipGetLastError();
 }
 
