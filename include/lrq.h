@@ -239,6 +239,11 @@ int64_t lrq_group_device_bytes(const void* host_table);
 /* writes the map of a device table whose first lrq_group_table_bytes() bytes
  * hold the uploaded host table (stream-ordered before this call) */
 int lrq_group_build_map(const void* host_table, void* device_table, lrq_stream_t stream);
+/* steps 3's copy and map of a table of at most LRQ_UPLOAD_TENSORS tensors in one
+ * launch (LRQ_ERR_CAPACITY for more): the host table travels as kernel arguments,
+ * so it need not be pinned, nor outlive the call */
+#define LRQ_UPLOAD_TENSORS 32
+int lrq_group_upload(const void* host_table, void* device_table, lrq_stream_t stream);
 int lrq_quant_grouped(const void* host_table, const void* device_table, lrq_stream_t stream);
 /* work-groups of a packed table's launch (for bandwidth accounting) */
 int64_t lrq_group_units(const void* host_table);

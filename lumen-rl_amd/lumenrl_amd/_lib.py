@@ -19,6 +19,7 @@ FMT_FP8_BLOCK, FMT_MXFP8, FMT_MXFP4, FMT_FP8_DEQUANT, FMT_TENSOR_SCALE, FMT_COPY
 FMT_CAST_E4M3, FMT_MXFP8_DEQUANT, FMT_MXFP4_DEQUANT = 6, 7, 8
 ERR_ARG, ERR_ALIGN, ERR_CAPACITY, ERR_TABLE = -1, -2, -3, -4
 STATIC_WORKSPACE_BYTES = 4 << 20  # LRQ_STATIC_WORKSPACE_BYTES
+UPLOAD_TENSORS = 32  # LRQ_UPLOAD_TENSORS
 
 
 class LrqError(RuntimeError):
@@ -58,6 +59,7 @@ SIGNATURES = {
     "lrq_group_kernel": (_CI, [_VP]),
     "lrq_group_device_bytes": (_I64, [_VP]),
     "lrq_group_build_map": (_CI, [_VP, _VP, _VP]),
+    "lrq_group_upload": (_CI, [_VP, _VP, _VP]),
     "lrq_group_workspace_bytes": (_I64, [_VP]),
     "lrq_tensor_scale_grouped": (_CI, [_VP, _VP, _VP, _I64, _VP]),
     "lrq_tensor_scale_grouped_static": (_CI, [_VP, _VP, _VP]),

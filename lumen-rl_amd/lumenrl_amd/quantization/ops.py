@@ -379,27 +379,34 @@ class _GroupLaunch:
         need = L.lrq_group_table_bytes(_FMTS[fmt], descs, n, in_dtype, br, bc, flags)
         if need < 0:
             _lib.check(int(need), "lrq_group_table_bytes")
-        self.host = torch.empty(int(need), dtype=torch.uint8, pin_memory=True)
+        small = n <= _lib.UPLOAD_TENSORS
+        self.host = torch.empty(int(need), dtype=torch.uint8, pin_memory=not small)
         rc = L.lrq_group_pack(_FMTS[fmt], descs, n, in_dtype, br, bc, flags,
                               self.host.data_ptr(), int(need))
         _lib.check(rc, "lrq_group_pack")
         # The device table is allocated and written on the caller's current
         # stream: stream-ordered like any torch op, so a recycled allocation
-        # is never overwritten while an earlier launch may still read it.  The
-        # copy is from pinned memory and does not block the host (a pageable
-        # copy would wait for the stream to drain, serializing plan building,
-        # e.g. every quantize_state_dict call, with the device).  Only the
-        # header and descriptors travel; the device writes the work-group map
-        # behind them itself (4 bytes per work-group: 8 MB for a whole 8B state).
+        # is never overwritten while an earlier launch may still read it.  A
+        # table of a few tensors travels as the arguments of the launch that
+        # writes it.  A longer one is copied from pinned memory, which does not
+        # block the host (a pageable copy would wait for the stream to drain,
+        # serializing plan building, e.g. every quantize_state_dict call, with
+        # the device): only the header and descriptors, and the device writes
+        # the work-group map behind them itself (4 bytes per work-group: 8 MB
+        # for a whole 8B state).
         dev_bytes = int(L.lrq_group_device_bytes(self.host.data_ptr()))
         if dev_bytes < 0:
             _lib.check(dev_bytes, "lrq_group_device_bytes")
         self.dev = torch.empty(dev_bytes, dtype=torch.uint8, device=device)
         with _on(device):
             self.home = torch.cuda.current_stream(device)
-            self.dev[: int(need)].copy_(self.host, non_blocking=True)
-            rc = L.lrq_group_build_map(self.host.data_ptr(), self.dev.data_ptr(), _stream(device))
-            _lib.check(rc, "lrq_group_build_map")
+            if small:
+                rc = L.lrq_group_upload(self.host.data_ptr(), self.dev.data_ptr(), _stream(device))
+                _lib.check(rc, "lrq_group_upload")
+            else:
+                self.dev[: int(need)].copy_(self.host, non_blocking=True)
+                rc = L.lrq_group_build_map(self.host.data_ptr(), self.dev.data_ptr(), _stream(device))
+                _lib.check(rc, "lrq_group_build_map")
             self.ready = torch.cuda.Event()
             self.ready.record(self.home)
         self.device = device

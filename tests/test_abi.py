@@ -578,3 +578,15 @@ def test_fp8_linear_arguments_are_checked_before_any_device_call():
     for bad in ({"x": odd}, {"codes": ctypes.c_void_p(0x10008)}, {"scales": odd}, {"out": ctypes.c_void_p(0x10004)},
                 {"bias": odd}):
         assert call(**bad) == _lib.ERR_ALIGN, bad
+
+
+def test_table_upload_checks_its_arguments_before_any_device_call():
+    small, big = _pack(_lib.FMT_FP8_BLOCK, QWEN3_8B_LAYER), _pack(_lib.FMT_FP8_BLOCK, QWEN3_8B_LAYER * 5)
+    dev = ctypes.c_void_p(0x1000)
+    assert L().lrq_group_upload(None, dev, None) == _lib.ERR_ARG
+    assert L().lrq_group_upload(small.ctypes.data, None, None) == _lib.ERR_ARG
+    assert L().lrq_group_upload(small.ctypes.data, ctypes.c_void_p(0x1040), None) == _lib.ERR_ALIGN
+    assert L().lrq_group_upload(big.ctypes.data, dev, None) == _lib.ERR_CAPACITY  # 35 tensors
+    junk = np.zeros(4096, np.uint8)
+    assert L().lrq_group_upload(junk.ctypes.data, dev, None) == _lib.ERR_TABLE
+    assert re.search(r"#define LRQ_UPLOAD_TENSORS (\d+)", open(HEADER).read()).group(1) == str(_lib.UPLOAD_TENSORS)
