@@ -107,7 +107,7 @@ def _scaled(tensors: dict[str, torch.Tensor], block: tuple[int, int],
     """Blockwise FP8 + ``<name>_scale_inv`` for accepted tensors, the rest kept."""
 
     def quantize(xs: list[torch.Tensor]) -> list[tuple[torch.Tensor, torch.Tensor]]:
-        launches = ops.ChunkedLaunches(lambda ys: ops.QuantPlan(ys, "fp8_block", block).run())
+        launches = ops.ChunkedLaunches(lambda ys: ops.QuantPlan(ys, "fp8_block", block).run_new())
         done: dict[int, tuple[torch.Tensor, torch.Tensor]] = {}
         for i, t in enumerate(xs):
             x = _kernel_input(t, t.device)

@@ -73,8 +73,45 @@ def _kernel_dtype(w: Tensor) -> torch.dtype:
     return torch.float32 if w.dtype == torch.float64 else w.dtype
 
 
-def _signature(ws: list[Tensor]) -> tuple:
-    return tuple((w.device, w.dtype, tuple(w.shape), tuple(w.stride()), w.data_ptr()) for w in ws)
+def _signature(w: Tensor) -> tuple:
+    """What the plan's table holds of a weight."""
+    return w.data_ptr(), w.shape, w.stride(), w.dtype, w.device
+
+
+def _projections(model: nn.Module) -> list[tuple[str, nn.Linear]]:
+    """(last name component, module) of every q/k/v projection, in the order and
+    with the names of ``model.named_modules()``: each module once, under the
+    first path that reaches it."""
+    found, seen = [], set()
+
+    def walk(module: nn.Module, short: str) -> None:
+        if module in seen:
+            return
+        seen.add(module)
+        if short in _KV_PROJECTIONS and isinstance(module, nn.Linear):
+            found.append((short, module))
+        for name, child in module._modules.items():
+            if child is None:
+                continue
+            if type(child).named_modules is not nn.Module.named_modules:
+                raise _OwnNames
+            walk(child, name.rpartition(".")[2])
+
+    try:
+        if type(model).named_modules is not nn.Module.named_modules:
+            raise _OwnNames
+        walk(model, "")
+    except _OwnNames:  # a module with a traversal of its own is asked for it
+        found = []
+        for name, module in model.named_modules():
+            short = name.rpartition(".")[2]
+            if isinstance(module, nn.Linear) and short in _KV_PROJECTIONS:
+                found.append((short, module))
+    return found
+
+
+class _OwnNames(Exception):
+    pass
 
 
 class FP8KVCacheQuantizer:
@@ -87,47 +124,48 @@ class FP8KVCacheQuantizer:
         if self._atom_spec is None:
             logger.debug("atom.quant_spec not available; KV cache path uses torch heuristics only.")
         self._groups: dict[torch.dtype, _ScaleGroup] = {}
-        self._signature: tuple = ()
+        self._signature: list[tuple] = []
+        self._slots: list[tuple[torch.dtype, int]] = []  # each weight's group and place in it
 
-    def _scales(self, weights: list[Tensor]) -> list[Tensor]:
-        """0-dim float32 device scales, one per weight, in order."""
-        sig = _signature(weights)
+    def _run(self, weights: list[Tensor]) -> dict[torch.dtype, Tensor]:
+        """Each group's scale vector, recomputed; weight i's is at ``_slots[i]``."""
+        sig = [_signature(w) for w in weights]
         if sig != self._signature:
+            weights = [w.detach() for w in weights]
             dev = next((w.device for w in weights if w.is_cuda), None) or ops.require_device()
             by_dtype: dict[torch.dtype, list[Tensor]] = {}
+            slots = []
             for w in weights:
-                by_dtype.setdefault(_kernel_dtype(w), []).append(w)
+                ws = by_dtype.setdefault(_kernel_dtype(w), [])
+                slots.append((_kernel_dtype(w), len(ws)))
+                ws.append(w)
             self._groups = {dt: _ScaleGroup(ws, dev) for dt, ws in by_dtype.items()}
+            self._slots = slots
             self._signature = sig
-        vecs = {dt: g.run() for dt, g in self._groups.items()}
-        taken = {dt: 0 for dt in vecs}
-        out = []
-        for w in weights:
-            dt = _kernel_dtype(w)
-            out.append(vecs[dt][taken[dt]])
-            taken[dt] += 1
-        return out
+        return {dt: g.run() for dt, g in self._groups.items()}
 
     def recalibrate_scales(self, model: nn.Module) -> None:
         """Recompute every q/k/v projection's scale from its current weight."""
         if not self._config.is_fp8_enabled():
             logger.debug("FP8 disabled; skipping KV scale recalibration.")
             return
-        targets = []
-        for name, module in model.named_modules():
-            short = name.rpartition(".")[2]
-            if isinstance(module, nn.Linear) and short in _KV_PROJECTIONS:
-                targets.append((short, module))
+        targets = _projections(model)
         if not targets:
             logger.warning("recalibrate_scales: no q_proj/k_proj/v_proj Linear layers found on model.")
             return
-        scales = self._scales([m.weight.detach() for _, m in targets])
-        for (short, module), s in zip(targets, scales):
+        vecs = self._run([m.weight for _, m in targets])
+        base = {dt: (v.data_ptr(), v.device) for dt, v in vecs.items()}
+        for (short, module), (dt, i) in zip(targets, self._slots):
             name = _BUFFER_PREFIX + short
-            if hasattr(module, name):
+            buf = module._buffers.get(name)
+            if buf is None and hasattr(module, name):
                 buf = getattr(module, name)
-                if not (isinstance(buf, Tensor) and buf.device == s.device and buf.data_ptr() == s.data_ptr()):
-                    buf.copy_(s.to(buf.device))
+            at, dev = base[dt]
+            if isinstance(buf, Tensor) and buf.data_ptr() == at + 4 * i and buf.device == dev:
+                continue  # a view of the vector the kernels have just written
+            s = vecs[dt][i]
+            if name in module._buffers or hasattr(module, name):
+                buf.copy_(s.to(buf.device))
             else:
                 home = module.weight.device
                 module.register_buffer(name, s if home == s.device else s.to(home))

@@ -27,6 +27,7 @@ from lumenrl_amd import _lib
 _IN_DTYPES = {torch.bfloat16: _lib.DTYPE_BF16, torch.float16: _lib.DTYPE_F16,
               torch.float32: _lib.DTYPE_F32}
 _ESIZE = {torch.bfloat16: 2, torch.float16: 2, torch.float32: 4}
+_SIZE = {**_ESIZE, torch.float64: 8, torch.uint8: 1}
 
 
 def require_device() -> torch.device:
@@ -39,21 +40,40 @@ def require_device() -> torch.device:
     return torch.device("cuda", torch.cuda.current_device())
 
 
+# torch's own bindings, without the Python wrappers' lazy-initialization checks
+# (a device tensor exists wherever these are called)
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_current_device = getattr(torch._C, "_cuda_getDevice", None) or torch.cuda.current_device
+_capturing = getattr(torch._C, "_cuda_isCurrentStreamCapturing", None) or torch.cuda.is_current_stream_capturing
+_STAY = contextlib.nullcontext()
 
 
-def _stream(device: torch.device) -> ctypes.c_void_p:
-    """The current torch stream of ``device`` as a hipStream_t."""
+def _stream(device: torch.device) -> int:
+    """The current torch stream of ``device`` as a hipStream_t (its address)."""
     if _raw_stream is not None:
-        return ctypes.c_void_p(_raw_stream(device.index))
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+        return _raw_stream(device.index)
+    return torch.cuda.current_stream(device).cuda_stream
 
 
 def _on(device: torch.device):
     """Make ``device`` current for a launch; a no-op when it already is."""
-    if device.index == torch.cuda.current_device():
-        return contextlib.nullcontext()
+    if device.index == _current_device():
+        return _STAY
     return torch.cuda.device(device)
+
+
+def _dense(shape: tuple, dtype: torch.dtype, device: torch.device) -> Tensor:
+    """``torch.empty(shape)``: torch parses the strided form's arguments in two
+    thirds of the time, 1 us per output."""
+    if len(shape) == 2:
+        strides = (shape[1] or 1, 1)
+    else:
+        strides, n = [], 1
+        for d in reversed(shape):
+            strides.append(n)
+            n *= d or 1
+        strides.reverse()
+    return torch.empty_strided(shape, strides, dtype=dtype, device=device)
 
 
 def _check_input(x: Tensor, what: str, allow_f64: bool = False) -> None:
@@ -119,7 +139,7 @@ def fp8_block_quant(x: Tensor, block: tuple[int, int], *, native_arith: bool = F
     br, bc = int(block[0]), int(block[1])
     if br < 1 or bc < 1:
         raise ValueError(f"block must be positive, got {block}")
-    shape = x.shape if x.dim() >= 2 else (1,) + tuple(x.shape)
+    shape = tuple(x.shape) if x.dim() >= 2 else (1,) + tuple(x.shape)
     xm, batch, rows, cols, ld, bstride = matrix_view(x)
     native = native_arith and x.dtype != torch.float32
     flags = 0
@@ -135,18 +155,19 @@ def fp8_block_quant(x: Tensor, block: tuple[int, int], *, native_arith: bool = F
         sdt = torch.bfloat16
     else:
         raise ValueError(f"scale_dtype must be float32 or bfloat16, got {scale_dtype}")
-    codes = torch.empty(shape, dtype=torch.float8_e4m3fn, device=x.device)
-    sshape = tuple(shape[:-2]) + (-(-rows // br), -(-cols // bc))
-    scales = torch.empty(sshape, dtype=sdt, device=x.device)
+    dev = x.device
+    codes = _dense(shape, torch.float8_e4m3fn, dev)
+    scales = _dense(shape[:-2] + (-(-rows // br), -(-cols // bc)), sdt, dev)
     if x.dim() < 2:
         codes = codes.reshape(x.shape)
     if batch * rows * cols == 0:
         return codes, scales
-    with _on(x.device):
+    with _on(dev):
         rc = _lib.lib().lrq_fp8_block_quant(
             xm.data_ptr(), _IN_DTYPES.get(x.dtype, _lib.DTYPE_F64), batch, rows, cols, ld, bstride,
-            br, bc, codes.data_ptr(), scales.data_ptr(), flags, _stream(x.device))
-    _lib.check(rc, "lrq_fp8_block_quant")
+            br, bc, codes.data_ptr(), scales.data_ptr(), flags, _stream(dev))
+    if rc:
+        _lib.check(rc, "lrq_fp8_block_quant")
     return codes, scales
 
 
@@ -198,7 +219,7 @@ def act_qdq(x: Tensor, block: int = 128, *, pow2: bool = False,
     if xm.stride(-1) != 1:  # any row pitch and element alignment, but unit-stride rows
         xm = xm.contiguous()
     if out is None:
-        out = torch.empty((rows, last), dtype=torch.float32, device=x.device)
+        out = _dense((rows, last), torch.float32, x.device)
     elif (out.dtype != torch.float32 or tuple(out.shape) != (rows, last) or not out.is_contiguous()
           or out.device != x.device):
         raise ValueError(f"act_qdq: out must be a contiguous float32 {(rows, last)} tensor on {x.device}")
@@ -238,22 +259,33 @@ def fp8_linear(x: Tensor, codes: Tensor, scales: Tensor, bias: Optional[Tensor] 
     if bias is not None and (tuple(bias.shape) != (n,) or bias.dtype not in _IN_DTYPES or bias.device != x.device
                              or not bias.is_contiguous()):
         raise ValueError(f"fp8_linear: bias must be a contiguous [{n}] tensor on {x.device}")
-    rows = x.numel() // last if last else 0
-    xm = x.reshape(rows, last)
-    if xm.stride(-1) != 1:  # as act_qdq: any row pitch and element alignment, but unit-stride rows
-        xm = xm.contiguous()
-    out = torch.empty((rows, n), dtype=x.dtype, device=x.device)
-    if out.numel() == 0:
+    return fp8_linear_checked(x, codes, scales, bias)
+
+
+def fp8_linear_checked(x: Tensor, codes: Tensor, scales: Tensor, bias: Optional[Tensor]) -> Tensor:
+    """``fp8_linear`` of operands the caller has already checked."""
+    n, k = codes.shape
+    if x.dim() == 2 and x.is_contiguous():
+        xm, rows, ld = x, x.shape[0], k
+    else:
+        rows = x.numel() // k if k else 0
+        xm = x.reshape(rows, k)
+        if xm.stride(-1) != 1:  # as act_qdq: any row pitch and element alignment, but unit-stride rows
+            xm = xm.contiguous()
+        ld = xm.stride(0) if rows > 1 else k
+        if ld > FP8_LINEAR_MAX_PITCH:
+            xm, ld = xm.contiguous(), k
+    dev = x.device
+    out = _dense((rows, n), x.dtype, dev)
+    if rows == 0 or n == 0:
         return out
-    ld = xm.stride(0) if rows > 1 else last
-    if ld > FP8_LINEAR_MAX_PITCH:
-        xm, ld = xm.contiguous(), last
-    with _on(x.device):
+    with _on(dev):
         rc = _lib.lib().lrq_fp8_linear(xm.data_ptr(), _IN_DTYPES[x.dtype], rows, k, ld, codes.data_ptr(),
                                        scales.data_ptr(), n, bias.data_ptr() if bias is not None else None,
                                        _IN_DTYPES[bias.dtype] if bias is not None else 0, out.data_ptr(),
-                                       _stream(x.device))
-    _lib.check(rc, "lrq_fp8_linear")
+                                       _stream(dev))
+    if rc:
+        _lib.check(rc, "lrq_fp8_linear")
     return out
 
 
@@ -371,7 +403,7 @@ class _GroupLaunch:
                  flags: int, device: torch.device) -> None:
         L = _lib.lib()
         with _on(device):
-            if torch.cuda.is_current_stream_capturing():
+            if _capturing():
                 # a captured upload would re-read this plan's pinned table on every
                 # replay, after the plan (and its table) may be gone
                 raise RuntimeError("build lrq plans before HIP graph capture; capture only run()")
@@ -400,6 +432,7 @@ class _GroupLaunch:
         self.dev = torch.empty(dev_bytes, dtype=torch.uint8, device=device)
         with _on(device):
             self.home = torch.cuda.current_stream(device)
+            self.home_raw = _stream(device)
             if small:
                 rc = L.lrq_group_upload(self.host.data_ptr(), self.dev.data_ptr(), _stream(device))
                 _lib.check(rc, "lrq_group_upload")
@@ -416,23 +449,24 @@ class _GroupLaunch:
         # table's device address, so the table must live and stay unchanged.
         self.captured = False
 
-    def _enter(self) -> None:
+    def _enter(self, capturing: bool) -> None:
         """Order a launch on another stream after the table upload, and tell the
         allocator that stream uses the plan's buffers (so freeing the plan
         cannot recycle them under a running launch).  Inside a graph capture
         this is skipped: the upload was ordered by the uncaptured warm-up run
         that capture requires anyway."""
-        cur = torch.cuda.current_stream(self.device)
-        if cur == self.home or torch.cuda.is_current_stream_capturing():
+        if capturing or _stream(self.device) == self.home_raw:
             return
+        cur = torch.cuda.current_stream(self.device)
         cur.wait_event(self.ready)
         for b in self.buffers:
             b.record_stream(cur)
 
     def run(self) -> None:
         with _on(self.device):
-            self._enter()
-            self.captured |= torch.cuda.is_current_stream_capturing()
+            capturing = _capturing()
+            self.captured |= capturing
+            self._enter(capturing)
             rc = _lib.lib().lrq_quant_grouped(self.host.data_ptr(), self.dev.data_ptr(),
                                               _stream(self.device))
         _lib.check(rc, "lrq_quant_grouped")
@@ -442,8 +476,9 @@ class _GroupLaunch:
 
     def run_tensor_scale(self, workspace: Tensor) -> None:
         with _on(self.device):
-            self._enter()
-            self.captured |= torch.cuda.is_current_stream_capturing()
+            capturing = _capturing()
+            self.captured |= capturing
+            self._enter(capturing)
             rc = _lib.lib().lrq_tensor_scale_grouped(self.host.data_ptr(), self.dev.data_ptr(),
                                                      workspace.data_ptr(), _nbytes(workspace),
                                                      _stream(self.device))
@@ -451,8 +486,9 @@ class _GroupLaunch:
 
     def run_tensor_scale_static(self) -> None:
         with _on(self.device):
-            self._enter()
-            self.captured |= torch.cuda.is_current_stream_capturing()
+            capturing = _capturing()
+            self.captured |= capturing
+            self._enter(capturing)
             rc = _lib.lib().lrq_tensor_scale_grouped_static(self.host.data_ptr(), self.dev.data_ptr(),
                                                             _stream(self.device))
         _lib.check(rc, "lrq_tensor_scale_grouped_static")
@@ -493,8 +529,9 @@ class _GroupLaunches:
     def __init__(self, fmt: str, descs, sizes: Sequence[int], in_dtype: int, block: tuple[int, int],
                  flags: int, device: torch.device, buffers: Optional[Sequence[Sequence[Tensor]]] = None) -> None:
         self.parts: list[_GroupLaunch] = []
-        for i, j in launch_ranges(sizes):
-            sub = (_lib.LrqTensor * (j - i))(*descs[i:j])
+        ranges = launch_ranges(sizes)
+        for i, j in ranges:
+            sub = descs if j - i == len(sizes) else (_lib.LrqTensor * (j - i))(*descs[i:j])
             part = _GroupLaunch(fmt, sub, j - i, in_dtype, block, flags, device)
             if buffers is not None:
                 part.buffers += [b for k in range(i, j) for b in buffers[k]]
@@ -502,11 +539,11 @@ class _GroupLaunches:
         # One kernel for the whole list, as one table requires of its tensors,
         # wherever the launches split it: the first tensor of the first part
         # whose kernel differs is the first tensor that differs from tensor 0.
-        kinds = [int(_lib.lib().lrq_group_kernel(p.host.data_ptr())) for p in self.parts]
+        kinds = [int(_lib.lib().lrq_group_kernel(p.host.data_ptr())) for p in self.parts] if len(ranges) > 1 else []
         for k in kinds:
             if k < 0:
                 _lib.check(k, "lrq_group_kernel")
-        for (i, _), k in zip(launch_ranges(sizes), kinds):
+        for (i, _), k in zip(ranges, kinds):
             if k != kinds[0]:
                 raise ValueError(f"tensor {i} needs a different kernel than tensor 0 "
                                  "(alignment/shape); group it separately")
@@ -724,7 +761,8 @@ class QuantPlan:
         dt = tensors[0].dtype
         dev = tensors[0].device
         for t in tensors:
-            _check_input(t, "QuantPlan", allow_f64=True)
+            if not (isinstance(t, Tensor) and t.is_cuda and (t.dtype in _IN_DTYPES or t.dtype == torch.float64)):
+                _check_input(t, "QuantPlan", allow_f64=True)
             if t.dtype != dt or t.device != dev:
                 raise ValueError("all tensors of a QuantPlan must share dtype and device")
         if dt == torch.float64 and not (fmt == "fp8_block" and native_arith):
@@ -750,34 +788,38 @@ class QuantPlan:
         self._flags = flags
         self._owned = outputs is None
         self._shapes = [tuple(t.shape) for t in tensors]
-        nbytes = 0
-        for i, t in enumerate(tensors):
-            shape = tuple(t.shape) if t.dim() >= 2 else (1,) + tuple(t.shape)
-            *_, rows, cols = shape
-            if fmt == "fp8_block":
-                cshape, cdt = shape, torch.float8_e4m3fn
-                sdt = dt if native else (torch.bfloat16 if flags & _lib.FLAG_SCALE_BF16 else torch.float32)
-                sshape = shape[:-2] + (-(-rows // br), -(-cols // bc))
-            else:
+        mx = fmt != "fp8_block"
+        cdt = torch.uint8 if fmt == "mxfp4" else torch.float8_e4m3fn
+        sdt = torch.uint8 if mx else dt if native else torch.bfloat16 if flags & _lib.FLAG_SCALE_BF16 else torch.float32
+        in_size, scale_size = tensors[0].element_size(), _SIZE[sdt]
+        self._sizes: list[int] = []  # algorithmic bytes of each tensor
+        for i, shape in enumerate(self._shapes):
+            if len(shape) < 2:
+                shape = (1,) + shape
+            lead, rows, cols = shape[:-2], shape[-2], shape[-1]
+            if mx:
                 if cols % 32:
                     raise ValueError(f"tensor {i}: last dim {cols} is not a multiple of 32")
-                lead = shape[:-1]
-                cshape = shape if fmt == "mxfp8" else lead + (cols // 2,)
-                cdt = torch.float8_e4m3fn if fmt == "mxfp8" else torch.uint8
-                sshape, sdt = lead + (cols // 32,), torch.uint8
+                cshape = shape if fmt == "mxfp8" else shape[:-1] + (cols // 2,)
+                sshape = shape[:-1] + (cols // 32,)
+            else:
+                cshape, sshape = shape, lead + (-(-rows // br), -(-cols // bc))
+            cells, n_scales = _prod(shape), _prod(sshape)
+            n_codes = cells // 2 if fmt == "mxfp4" else cells
             if outputs is None:
-                codes = torch.empty(cshape, dtype=cdt, device=dev)
-                scales = torch.empty(sshape, dtype=sdt, device=dev)
+                codes = _dense(cshape, cdt, dev)
+                scales = _dense(sshape, sdt, dev)
             else:
                 codes, scales = outputs[i]
-                if (codes.numel() * codes.element_size() != _prod(cshape)
-                        or scales.numel() * scales.element_size() != _prod(sshape) * _esize(sdt)
+                if (codes.numel() * codes.element_size() != n_codes
+                        or scales.numel() * scales.element_size() != n_scales * scale_size
                         or not codes.is_contiguous() or not scales.is_contiguous()
                         or codes.device != dev or scales.device != dev):
                     raise ValueError(f"output {i} must be contiguous device views of "
                                      f"{cshape} codes and {sshape} {sdt} scales")
             self.outputs.append((codes, scales))
-            nbytes += _nbytes(t) + _nbytes(codes) + _nbytes(scales)
+            self._sizes.append(cells * in_size + n_codes + n_scales * scale_size)
+        nbytes = sum(self._sizes)
         self.algorithmic_bytes = nbytes
         self._bind(list(tensors))
 
@@ -794,25 +836,28 @@ class QuantPlan:
                                "build (and capture) a new plan instead of re-binding this one")
         descs = (_lib.LrqTensor * len(tensors))()
         views = []
+        sig = []
         for i, (t, (codes, scales)) in enumerate(zip(tensors, self.outputs)):
             xm, batch, rows, cols, ld, bstride = matrix_view(t)
-            if xm.data_ptr() != t.data_ptr():
+            at = t.data_ptr()
+            if xm is not t and xm.data_ptr() != at:
                 raise ValueError(f"tensor {i} is not a strided matrix view; pass .contiguous()")
             views.append(xm)
-            descs[i].in_ = xm.data_ptr()
-            descs[i].codes = codes.data_ptr()
-            descs[i].scales = scales.data_ptr()
-            descs[i].batch, descs[i].rows, descs[i].cols = batch, rows, cols
-            descs[i].ld, descs[i].batch_stride = ld, bstride
-        sizes = [_nbytes(t) + _nbytes(c) + _nbytes(sc) for t, (c, sc) in zip(tensors, self.outputs)]
-        launch = _GroupLaunches(self.fmt, descs, sizes, _IN_DTYPES.get(self.dtype, _lib.DTYPE_F64),
+            descs[i] = (at, codes.data_ptr(), scales.data_ptr(), batch, rows, cols, ld, bstride)
+            sig.append((at, t.stride(), tuple(t.shape)))
+        launch = _GroupLaunches(self.fmt, descs, self._sizes, _IN_DTYPES.get(self.dtype, _lib.DTYPE_F64),
                                 self._block, self._flags, self.device,
                                 buffers=[list(pair) for pair in self.outputs] if self._owned else None)
         self._launch = launch
         self._views = views
         self.inputs = tensors
-        self._sig = [(t.data_ptr(), t.stride(), tuple(t.shape)) for t in tensors]
+        self._sig = sig
         self.units = launch.units
+
+    def run_new(self) -> list[tuple[Tensor, Tensor]]:
+        """``run()`` of a plan built just now: its inputs are where its table says."""
+        self._launch.run()
+        return self.outputs
 
     def run(self, inputs: Optional[Sequence[Tensor]] = None) -> list[tuple[Tensor, Tensor]]:
         """Enqueue the launch on the current stream; returns the (codes, scales) list.
@@ -881,7 +926,8 @@ class DequantPlan:
         descs = (_lib.LrqTensor * len(pairs))()
         self.inputs = []
         self.outputs: list[Tensor] = []
-        nbytes = 0
+        sizes = []
+        out_size, scale_size = (4 if out_dtype == torch.float32 else 2), _SIZE[sdt]
         for i, (c, sc) in enumerate(pairs):
             if c.dtype not in (torch.float8_e4m3fn, torch.uint8) or not c.is_cuda or not c.is_contiguous():
                 raise ValueError(f"pair {i}: codes must be contiguous float8_e4m3fn device tensors")
@@ -893,18 +939,13 @@ class DequantPlan:
             need = batch * (-(-rows // br)) * (-(-cols // bc))
             if sc.numel() != need:
                 raise ValueError(f"pair {i}: scales have {sc.numel()} elements, blocks need {need}")
-            out = torch.empty(c.shape, dtype=out_dtype, device=dev)
+            out = _dense(tuple(c.shape), out_dtype, dev)
             self.inputs.append((c, sc))
             self.outputs.append(out)
-            descs[i].in_ = c.data_ptr()
-            descs[i].codes = out.data_ptr()
-            descs[i].scales = sc.data_ptr()
-            descs[i].batch, descs[i].rows, descs[i].cols = batch, rows, cols
-            descs[i].ld, descs[i].batch_stride = cols, rows * cols
-            nbytes += _nbytes(c) + _nbytes(sc) + _nbytes(out)
-        self.algorithmic_bytes = nbytes
+            descs[i] = (c.data_ptr(), out.data_ptr(), sc.data_ptr(), batch, rows, cols, cols, rows * cols)
+            sizes.append(batch * rows * cols * (1 + out_size) + need * scale_size)
+        self.algorithmic_bytes = sum(sizes)
         flags = _lib.FLAG_OUT_BF16 if out_dtype == torch.bfloat16 else 0
-        sizes = [_nbytes(c) + _nbytes(sc) + _nbytes(o) for (c, sc), o in zip(self.inputs, self.outputs)]
         self._launch = _GroupLaunches("fp8_dequant", descs, sizes, _IN_DTYPES[sdt], (br, bc), flags, dev,
                                       buffers=[[o] for o in self.outputs])
         self.units = self._launch.units
@@ -1065,14 +1106,11 @@ class CastPlan:
             _check_input(t, "CastPlan")
             if t.dtype != dt or t.device != dev or not t.is_contiguous():
                 raise ValueError(f"tensor {i}: CastPlan needs contiguous {dt} tensors on {dev}")
-            out = torch.empty(t.shape, dtype=torch.float8_e4m3fn, device=dev)
+            out = _dense(tuple(t.shape), torch.float8_e4m3fn, dev)
             self.outputs.append(out)
-            descs[i].in_ = t.data_ptr()
-            descs[i].codes = out.data_ptr()
-            descs[i].scales = None
-            descs[i].batch, descs[i].rows, descs[i].cols = 1, 1, t.numel()
-            descs[i].ld, descs[i].batch_stride = t.numel(), t.numel()
-            nbytes += _nbytes(t) + _nbytes(out)
+            n = t.numel()
+            descs[i] = (t.data_ptr(), out.data_ptr(), None, 1, 1, n, n, n)
+            nbytes += n * (t.element_size() + 1)
         self.algorithmic_bytes = nbytes
         self._launch = _GroupLaunch("cast_e4m3", descs, len(tensors), _IN_DTYPES[dt], (1, 1), 0, dev)
         self._launch.buffers += self.outputs
@@ -1088,7 +1126,3 @@ def _prod(shape) -> int:
     for d in shape:
         p *= int(d)
     return p
-
-
-def _esize(dtype: torch.dtype) -> int:
-    return torch.empty((), dtype=dtype).element_size()

@@ -155,7 +155,7 @@ class WeightQuantizer:
         def quantize(xs: list[Tensor]) -> list[tuple[Tensor, Tensor]]:
             launches = ops.ChunkedLaunches(
                 lambda ys: ops.QuantPlan(ys, "fp8_block", (1, 128), use_pow2_scale=pow2,
-                                         scale_dtype=torch.bfloat16).run())
+                                         scale_dtype=torch.bfloat16).run_new())
             done: dict[int, tuple[Tensor, Tensor]] = {}
             for i, x in enumerate(xs):
                 if x.dtype == torch.float64:

@@ -126,8 +126,8 @@ def test_module_routes(monkeypatch):
     """The one-launch path where it applies; F.linear where autocast, the bias's
     gradient, another block, type or device need it, with the results it gives."""
     calls = []
-    real = ops.fp8_linear
-    monkeypatch.setattr(ops, "fp8_linear", lambda *a: calls.append(1) or real(*a))
+    real = ops.fp8_linear_checked
+    monkeypatch.setattr(ops, "fp8_linear_checked", lambda *a: calls.append(1) or real(*a))
     torch.manual_seed(1)
     mod, x = module(1024, 512, torch.bfloat16), torch.randn(2, 9, 512, device=DEV, dtype=torch.bfloat16)
 
