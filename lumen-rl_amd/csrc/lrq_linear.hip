@@ -32,8 +32,14 @@ typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-// 16 bytes of a 2-byte-aligned row, cached (x is read by many work-groups).
-__device__ __forceinline__ v4u load_x16(const void* p) { return *(const LRQ_GLOBAL v4u_in*)p; }
+// 16 bytes at a 32-bit offset from a wave-uniform base, from any 2-byte-aligned
+// address; cached, or past the caches for what one work-group reads once.
+typedef const LRQ_GLOBAL uint8_t* GlobalBytes;
+__device__ __forceinline__ v4u load_x16(GlobalBytes p, uint32_t off) { return *(const LRQ_GLOBAL v4u_in*)(p + off); }
+__device__ __forceinline__ v4u load_x16_nt(GlobalBytes p, uint32_t off) {
+  return __builtin_nontemporal_load((const LRQ_GLOBAL v4u_in*)(p + off));
+}
+__device__ __forceinline__ uint32_t load_scale16(GlobalBytes p, uint32_t off) { return *(const LRQ_GLOBAL uint16_t*)(p + off); }
 
 template <int DT>
 __device__ __forceinline__ float x16_to_f32(uint16_t b) {
@@ -84,7 +90,7 @@ __device__ __forceinline__ bool linear_nonfinite(const uint16_t* x, const uint16
   constexpr uint32_t kInf = DT == kBF16 ? 0x7F80u : 0x7C00u;
   bool bad = false;
   for (int i = 0; i < k && !bad; i += 8) {
-    const v4u v = load_x16(x + i);
+    const v4u v = load_x16((GlobalBytes)(x + i), 0);
     const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
     for (int j = 0; j < 4; ++j) bad |= (w[j] & 0x7FFFu) >= kInf || ((w[j] >> 16) & 0x7FFFu) >= kInf;
@@ -170,9 +176,9 @@ __global__ __launch_bounds__(64 * KW) void k_linear_rows(LinearArgs a) {
   uint8_t* const lx = lw + NT * 2048;
   // Tile bases in scalar registers and 32-bit offsets per lane.  Rows past the
   // end read the last one again; their sums are not stored.
-  const uint8_t* const w0 = a.codes + (int64_t)n0 * a.k;
-  const uint16_t* const s0 = a.scales + (int64_t)n0 * kb_n;
-  const uint8_t* const x0 = static_cast<const uint8_t*>(a.x) + 2 * (m0 * a.ldx);
+  const GlobalBytes w0 = (GlobalBytes)a.codes + (int64_t)n0 * a.k;
+  const GlobalBytes s0 = (GlobalBytes)a.scales + 2 * ((int64_t)n0 * kb_n);
+  const GlobalBytes x0 = (GlobalBytes)a.x + 2 * (m0 * a.ldx);
   uint32_t wo[NT][2], so[NT], xo[MT][4];
 #pragma unroll
   for (int j = 0; j < NT; ++j) {
@@ -182,7 +188,7 @@ __global__ __launch_bounds__(64 * KW) void k_linear_rows(LinearArgs a) {
       wo[j][h] = (uint32_t)(r < n_last ? r : n_last) * (uint32_t)a.k + 16 * (lane & 7);
     }
     const int r = 16 * j + c;
-    so[j] = (uint32_t)(r < n_last ? r : n_last) * (uint32_t)kb_n;
+    so[j] = (uint32_t)(r < n_last ? r : n_last) * (uint32_t)(2 * kb_n);
   }
 #pragma unroll
   for (int i = 0; i < MT; ++i)
@@ -198,18 +204,17 @@ __global__ __launch_bounds__(64 * KW) void k_linear_rows(LinearArgs a) {
   auto load = [&](LinStage<NT, MT>& st, int t) {
     const int kt = wave * steps + t, kb = kt < kb_n ? kt : kb_n - 1;
     const uint32_t keep = kt < kb_n ? 0xFFFFu : 0u;
-    const uint8_t* const wb = w0 + kb * kLinBlock;
-    const uint8_t* const xb = x0 + 2 * (kb * kLinBlock);
+    const GlobalBytes wb = w0 + kb * kLinBlock, xb = x0 + 2 * (kb * kLinBlock), sb = s0 + 2 * kb;
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
-      st.w[j][0] = ONCE ? load_nt(wb + wo[j][0]) : load_x16(wb + wo[j][0]);
-      st.w[j][1] = ONCE ? load_nt(wb + wo[j][1]) : load_x16(wb + wo[j][1]);
-      st.s[j] = gld<uint16_t>(s0 + kb + so[j]) & keep;
+      st.w[j][0] = ONCE ? load_x16_nt(wb, wo[j][0]) : load_x16(wb, wo[j][0]);
+      st.w[j][1] = ONCE ? load_x16_nt(wb, wo[j][1]) : load_x16(wb, wo[j][1]);
+      st.s[j] = load_scale16(sb, so[j]) & keep;
     }
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) st.x[i][q] = load_x16(xb + xo[i][q]);
+      for (int q = 0; q < 4; ++q) st.x[i][q] = load_x16(xb, xo[i][q]);
   };
   f32x4 acc[MT][NT];
 #pragma unroll
@@ -310,13 +315,14 @@ __global__ __launch_bounds__(64 * KW) void k_linear_rows(LinearArgs a) {
 // 4 x 4 x (2 x 4): 128 x 256 tiles, one work-group of 8 waves on a CU, two to a
 // SIMD, so that one's vector instructions and waits fall beside the other's
 // matrix instructions (4 waves of 128 x 64 each: 0.90 ms instead of 0.80).
-// 8192 tokens x [12288, 4096] take 0.80 ms (1035 TFLOP/s, matrix cores 47 % busy
+// 8192 tokens x [12288, 4096] take 0.79 ms (1046 TFLOP/s, matrix cores 47 % busy
 // at 1.9 GHz), 5.6 ms before by way of float32 operands and a float32 library
 // product (147 TFLOP/s).
 // The smaller tiles are for grids that would leave CUs idle with the large one:
 // each CU does less work per byte that passes its LDS, 28 us for 512 tokens x
-// [4096, 4096] in 64 x 128 tiles (59 in 128 x 256), 113 us for 1024 x [12288,
-// 4096] in 128 x 192 (125).
+// [4096, 4096] in 64 x 128 tiles (59 in 128 x 256), 115 us for 1024 x [12288,
+// 4096] in 128 x 192 (140).  32 x 32 matrix instructions need 16 more registers
+// than there are (1.07 ms with spills; 4 waves 0.96 ms).
 //
 // The compiler keeps the matrix instructions' results in vector registers
 // (-amdgpu-mfma-vgpr-form): in accumulation registers, its own choice here,
@@ -355,9 +361,9 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void k_linear_tiles(LinearArgs a, 
   const int m0 = tm * BM, n0 = tn * BN;
   const int n_last = (int)a.n - 1 - n0, m_last = (int)a.m - 1 - m0;
   const int kb_n = (int)(a.k / kLinBlock);
-  const uint8_t* const w0 = a.codes + (int64_t)n0 * a.k;
-  const uint16_t* const s0 = a.scales + (int64_t)n0 * kb_n;
-  const uint8_t* const x0 = static_cast<const uint8_t*>(a.x) + 2 * (m0 * a.ldx);
+  const GlobalBytes w0 = (GlobalBytes)a.codes + (int64_t)n0 * a.k;
+  const GlobalBytes s0 = (GlobalBytes)a.scales + 2 * ((int64_t)n0 * kb_n);
+  const GlobalBytes x0 = (GlobalBytes)a.x + 2 * (m0 * a.ldx);
   uint32_t xo[PA], wo[PB];
 #pragma unroll
   for (int p = 0; p < PA; ++p) {
@@ -370,23 +376,31 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void k_linear_tiles(LinearArgs a, 
     wo[p] = (uint32_t)(r < n_last ? r : n_last) * (uint32_t)a.k + 16 * (tid & 7);
   }
   const int sr = tid < BN ? tid : BN - 1;  // the scale this thread moves
-  const uint32_t so = (uint32_t)(sr < n_last ? sr : n_last) * (uint32_t)kb_n;
+  const uint32_t so = (uint32_t)(sr < n_last ? sr : n_last) * (uint32_t)(2 * kb_n);
   v4u gx[PA], gw[PB];
   uint32_t gs;
   // The moves of a block are spread over the tiles j = 0 .. FN - 2 of the block
   // before: stores into LDS in the first half, loads in the second.
   constexpr int HP = (FN - 1) / 2, HF = FN - 1 - HP;
+  // Keeps the widening of a loop-invariant offset at its load: hoisted out of the
+  // loop, as the compiler would, it costs two registers and a 64-bit addition at
+  // each load.  64 x 128 tiles come to 125 registers, so that two fit a CU (1075
+  // instead of 1190 us for 8192 tokens x [12288, 4096]); the largest tile, one on
+  // a CU either way, is 2 % faster without.
+  auto here = [](uint32_t off) {
+    if constexpr (FM * FN < 16) asm volatile("" : "+v"(off));
+    return off;
+  };
   auto fetch = [&](int kb, int j) {
     kb = kb < kb_n ? kb : kb_n - 1;
-    const uint8_t* const xb = x0 + 2 * (kb * kLinBlock);
-    const uint8_t* const wb = w0 + kb * kLinBlock;
+    const GlobalBytes wb = w0 + kb * kLinBlock, xb = x0 + 2 * (kb * kLinBlock), sb = s0 + 2 * kb;
 #pragma unroll
     for (int p = 0; p < PA; ++p)
-      if (j == HP + p * HF / PA) gx[p] = load_x16(xb + xo[p]);
+      if (j == HP + p * HF / PA) gx[p] = load_x16(xb, here(xo[p]));
 #pragma unroll
     for (int p = 0; p < PB; ++p)
-      if (j == HP + p * HF / PB) gw[p] = load_x16(wb + wo[p]);
-    if (j == HP) gs = gld<uint16_t>(s0 + kb + so);
+      if (j == HP + p * HF / PB) gw[p] = load_x16(wb, here(wo[p]));
+    if (j == HP) gs = load_scale16(sb, here(so));
   };
   auto put = [&](uint8_t* buf, int j) {
 #pragma unroll
@@ -525,8 +539,8 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void k_linear_tiles(LinearArgs a, 
 //   * k_linear_rows: kLinearRows ns a round of 256 work-groups.  It grows with the
 //     bytes that a CU moves through its vector cache and LDS, 2 mt + nt units (x
 //     has two bytes an element); shapes past 8 waves' LDS do not pay any more;
-//   * k_linear_tiles: `each` ns a round of tiles, one on a CU, and `once` more;
-//     three 64 x 64 tiles fit a CU, 280 ns apiece and 457 once.
+//   * k_linear_tiles: `each` ns for each 256 tiles, and `once` more; of 64 x 64
+//     tiles, three fit a CU, 280 ns and 457 once where they do.
 // From sweeps over all shapes at 1 to 8192 tokens and weights of [500 to 12288,
 // 1024 to 12288], where the shape it takes is 1 % from the fastest in the mean.
 constexpr int kLinearRows[3][4] = {{136, 190, 315, 380}, {165, 280, 400, 465}, {290, 380, 485, INT32_MAX}};
@@ -534,7 +548,7 @@ struct LinearTile {
   int m, n, each, once;
 };
 constexpr LinearTile kLinearTiles[] = {
-    {128, 256, 2075, -200}, {128, 192, 1720, -80}, {128, 128, 1330, -100}, {64, 128, 800, 75}, {64, 64, 398, 0}};
+    {128, 256, 2060, -190}, {128, 192, 1680, -80}, {128, 128, 1290, -60}, {64, 128, 670, 205}, {64, 64, 398, 0}};
 constexpr int kLinearTileKinds = sizeof(kLinearTiles) / sizeof(kLinearTiles[0]);
 struct LinearShape {
   int tile;    // index into kLinearTiles, or -1: k_linear_rows
