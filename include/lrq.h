@@ -161,8 +161,8 @@ int lrq_act_qdq(const void* in, int in_dtype, int64_t rows, int64_t cols, int64_
  *   codes  : [n, k] e4m3 bytes, dense;  scales : [n, k/128] bf16, dense;
  *   bias   : [n] of bias_dtype (bf16, fp16 or fp32), or null;
  *   out    : [rows, n] of x's type, dense, 16-byte aligned.
- * k a multiple of 128; k and ld at most 2^24; rows and n below 2^31 and rows * n
- * below 2^37.
+ * k a multiple of 128; k and ld at most 2^24; rows at most 2^28, n 2^26 and rows * n
+ * 2^33.
  */
 int lrq_fp8_linear(const void* x, int x_dtype, int64_t rows, int64_t k, int64_t ld,
                    const uint8_t* codes, const void* scales, int64_t n, const void* bias,

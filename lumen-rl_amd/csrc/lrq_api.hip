@@ -664,8 +664,8 @@ int lrq_fp8_linear(const void* x, int x_dtype, int64_t rows, int64_t k, int64_t 
   if (bias && !valid_dtype(bias_dtype)) return fail(LRQ_ERR_ARG, "bad bias dtype %d", bias_dtype);
   if (rows < 0 || n < 0 || k < 0 || k % lrq::kLinBlock != 0)
     return fail(LRQ_ERR_ARG, "k (%lld) must be a multiple of 128", (long long)k);
-  if (rows > INT32_MAX || n > INT32_MAX || k > lrq::kLinPitchMax || ld > lrq::kLinPitchMax ||
-      lrq::linear_grid(rows, n) > (1 << 25))
+  if (rows > lrq::kLinRowsMax || n > lrq::kLinOutMax || k > lrq::kLinPitchMax || ld > lrq::kLinPitchMax ||
+      rows * n > lrq::kLinCellsMax)
     return fail(LRQ_ERR_ARG, "linear of %lld x %lld x %lld (pitch %lld) is too large", (long long)rows, (long long)n,
                 (long long)k, (long long)ld);
   if (rows == 0 || n == 0) return 0;

@@ -239,7 +239,10 @@ hipError_t launch_act(const void* in, int dtype, int64_t rows, int64_t cols, int
 // transpose of the dequantized weight [n, k] (dense e4m3 codes, bf16 scales
 // [n, k / kLinBlock]), plus an optional bias [n]; y has x's 16-bit type.
 constexpr int64_t kLinBlock = 128;
-constexpr int64_t kLinPitchMax = 1 << 24; // row pitches: 32-bit byte offsets within a tile of rows
+constexpr int64_t kLinPitchMax = 1 << 24;  // row pitches: 32-bit byte offsets within a tile of 256 rows
+// m, n and m * n: fewer than 2^23 of the smallest (64 x 64) tiles, so fewer than
+// 2^32 threads, and as few in a grid of 16-row groups
+constexpr int64_t kLinRowsMax = 1 << 28, kLinOutMax = 1 << 26, kLinCellsMax = int64_t(1) << 33;
 struct LinearArgs {
   const void* x;
   const uint8_t* codes;
@@ -249,7 +252,6 @@ struct LinearArgs {
   int64_t ldx, m, n, k;
   int bias_dtype;
 };
-int64_t linear_grid(int64_t m, int64_t n);  // work-groups at most, but for few tokens
 hipError_t launch_linear(const LinearArgs& a, int dtype, hipStream_t stream);
 
 // Diagnostics: element encoders applied to raw inputs.

@@ -614,9 +614,6 @@ static void launch_linear_dt(const LinearArgs& a, const LinearShape& s, hipStrea
   }
 }
 
-// Work-groups of the smallest tile: the host refuses grids past 2^24 / 2.
-int64_t linear_grid(int64_t m, int64_t n) { return ceil_div(m, 64) * ceil_div(n, 64); }
-
 hipError_t launch_linear(const LinearArgs& a, int dtype, hipStream_t stream) {
   const LinearShape s = linear_shape(a.m, a.n);
   if (dtype == kBF16) launch_linear_dt<kBF16>(a, s, stream);

@@ -235,7 +235,8 @@ def act_qdq(x: Tensor, block: int = 128, *, pow2: bool = False,
 
 
 FP8_LINEAR_MAX_PITCH = 1 << 24  # fp8_linear: K, and the row pitch the kernels read x with
-FP8_LINEAR_MAX_CELLS = 1 << 36  # fp8_linear: tokens * out_features
+FP8_LINEAR_MAX_TOKENS, FP8_LINEAR_MAX_OUT = 1 << 28, 1 << 26
+FP8_LINEAR_MAX_CELLS = 1 << 33  # fp8_linear: tokens * out_features
 
 
 def fp8_linear(x: Tensor, codes: Tensor, scales: Tensor, bias: Optional[Tensor] = None) -> Tensor:

@@ -572,7 +572,7 @@ def test_fp8_linear_arguments_are_checked_before_any_device_call():
 
     assert call(rows=0) == 0 and call(n=0) == 0
     for bad in ({"dt": 2}, {"dt": 7}, {"k": 200}, {"k": 0}, {"ld": 255}, {"ld": 0}, {"rows": -1}, {"n": -1},
-                {"rows": 1 << 31}, {"rows": 1 << 20, "n": 1 << 18}, {"n": 1 << 31}, {"k": (1 << 24) + 128, "ld": 1 << 25}, {"ld": (1 << 24) + 1},
+                {"rows": (1 << 28) + 1}, {"rows": 1 << 20, "n": (1 << 13) + 1}, {"n": (1 << 26) + 1}, {"k": (1 << 24) + 128, "ld": 1 << 25}, {"ld": (1 << 24) + 1},
                 {"x": None}, {"codes": None}, {"scales": None}, {"out": None}, {"bias": fake, "bdt": 3}):
         assert call(**bad) == _lib.ERR_ARG, bad
     for bad in ({"x": odd}, {"codes": ctypes.c_void_p(0x10008)}, {"scales": odd}, {"out": ctypes.c_void_p(0x10004)},
