@@ -84,7 +84,12 @@ __device__ __forceinline__ uint32_t abs_max(const float (&x)[N]) {
 // 8t..8t+7 of the wave's 512-element span; the float32 results are exchanged
 // across the wave so that store h of lane t writes elements 256h + 4t .. +3
 // (owned by lane 32h + t/2, half t&1): each store instruction writes 1 KiB
-// of whole cache lines.
+// of whole cache lines.  The loads go through the caches, unlike a weight's: an
+// activation was written just before and is read again.  [8192, 4096] bf16 with
+// 67 MB inputs in turn, 201 MB in all: 28.8 us (7.0 TB/s), 32.6 with nontemporal
+// loads; [8192, 12288], past the 256 MB memory-side cache: 92.1 and 92.5 us.
+// Stores that stay nontemporal (cached 33.5 us) and one chunk a lane (two 34 to
+// 39 us, four 37) are the better of those.
 template <int DT, int LPB, bool DENSE>
 __global__ __launch_bounds__(256) void k_act_qdq8(const uint16_t* __restrict__ in, int64_t rows, int64_t cols,
                                                   int64_t ld, float* __restrict__ out, int pow2) {
@@ -93,7 +98,7 @@ __global__ __launch_bounds__(256) void k_act_qdq8(const uint16_t* __restrict__ i
   const int64_t span = xcd_unit<kXcdRunStream>(blockIdx.x, gridDim.x) * 2048 + (threadIdx.x >> 6) * 512;
   const int64_t e = span + 8 * lane;
   v4u v = {0u, 0u, 0u, 0u};
-  if (e < n) v = load_nt(in + act_offset(e, cols, ld, DENSE));
+  if (e < n) v = load_live(in + act_offset(e, cols, ld, DENSE));
   const uint32_t w[4] = {v.x, v.y, v.z, v.w};
   float x[8];
 #pragma unroll

@@ -294,6 +294,8 @@ typedef unsigned int v4u_in __attribute__((ext_vector_type(4), aligned(2)));
 __device__ __forceinline__ v4u load_nt(const void* p) {
   return __builtin_nontemporal_load((const LRQ_GLOBAL v4u_in*)p);
 }
+// The same through the caches, for data that was just written or is read again.
+__device__ __forceinline__ v4u load_live(const void* p) { return *(const LRQ_GLOBAL v4u_in*)p; }
 // Code loads of the dequant kernels take any byte alignment, likewise.
 typedef unsigned int v2u_in __attribute__((ext_vector_type(2), aligned(1)));
 typedef uint32_t u32_in __attribute__((aligned(1)));
