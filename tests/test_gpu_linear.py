@@ -162,6 +162,37 @@ def test_module_routes(monkeypatch):
         check(y, x[0, :1].half(), half.weight_fp8, half.weight_scale)
 
 
+def test_module_with_replaced_buffers():
+    """A bias or scales that do not have one value per row (or block) of the weight
+    go to the ops that check them: F.linear broadcasts one bias for all, and refuses
+    other lengths; the dequantization refuses scales that are too few.  A bias under
+    vmap is a batch of them."""
+    torch.manual_seed(2)
+    mod, x = module(1024, 512, torch.bfloat16), torch.randn(6, 512, device=DEV, dtype=torch.bfloat16)
+    codes, scales = mod.weight_fp8, mod.weight_scale
+    with torch.no_grad():
+        mod.bias = nn.Parameter(torch.full((1,), 0.5, device=DEV, dtype=torch.bfloat16))
+        check(mod(x), x, codes, scales, mod.bias.expand(1024))
+        mod.bias = nn.Parameter(torch.zeros(1000, device=DEV, dtype=torch.bfloat16))
+        with pytest.raises(RuntimeError):
+            mod(x)
+        mod.bias = None
+        mod.weight_scale = scales[:1000].contiguous()
+        with pytest.raises(ValueError):
+            mod(x)
+        mod.weight_scale = scales
+        batch = torch.randn(3, 1024, device=DEV, dtype=torch.bfloat16)
+
+        def with_bias(b):
+            mod.__dict__["bias"] = b
+            return mod(x)
+
+        del mod.bias
+        y = torch.vmap(with_bias)(batch)
+        for i in range(3):
+            check(y[i], x, codes, scales, batch[i])
+
+
 def test_linear_in_a_graph():
     """Captured and replayed with new inputs and eager work between the replays."""
     x, codes, scales = operands(8, 1024, 512, torch.bfloat16)
