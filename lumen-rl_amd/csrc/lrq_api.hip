@@ -179,6 +179,10 @@ bool plan_units(const LaunchCfg& cfg, Desc& d) {
       d.units_r = (d.rows + cfg.blk_r - 1) / cfg.blk_r;
       d.units_c = (d.cols + cfg.blk_c - 1) / cfg.blk_c;
       d.units = d.batch * d.units_r * d.units_c;
+      if (cfg.kernel == kKernTile128 && lrq::tile_band(cfg.in_dtype, d.cols, d.batch * d.units_r)) {
+        d.units_c = 1;
+        d.units = d.batch * d.units_r;
+      }
       if (cfg.kernel == kKernTile128) d.bpr = tile_run_log2(d.ld * esize(cfg.in_dtype));
       return true;
     case kKernF64Row: {  // 4 waves x f64_row_instr instructions of 128 doubles

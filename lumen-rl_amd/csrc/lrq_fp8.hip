@@ -136,8 +136,8 @@ __device__ __forceinline__ void store_scale(void* scales, int64_t idx, float s, 
 // again in place of those outside: they are in its amax anyway, so no load hangs
 // on a branch, and only the stores look at the edges.  Tiles of at most 64
 // columns take CPR = 8, two loads a thread instead of four with half the lanes
-// idle: 128 expert matrices of 2048 x 192 (tiles of 128 and of 64 columns) take
-// 28.9 us, 29.6 us with masked loads over 128 columns.
+// idle: 77 matrices of 2048 x 320 (the last tile of a row 64 wide) take 28.1 us,
+// 28.6 with masked loads over 128 columns, and 8 of 1000 x 192 4.5 us (6.9).
 template <int DT, int CDT, int T, int CPR, bool FULL>
 __device__ __forceinline__ void tile_body(const Desc& d, int64_t b, int64_t r0, int64_t c0, int64_t u, int pow2,
                                           int scale_bf16, uint32_t* red) {
@@ -187,11 +187,70 @@ __device__ __forceinline__ void tile_body(const Desc& d, int64_t b, int64_t r0, 
   }
 }
 
+// Both tiles of a row band of 128 < cols <= 192 (cpr = cols / 8 chunks a row), 16-bit
+// input.  The chunks are taken in memory order, so each wave instruction reads 1 KiB
+// and writes 512 bytes in a row: one work-group per tile reads runs of 256 bytes and
+// of the rest, and writes parts of lines at most rows.  128 expert matrices of 2048 x
+// 192: 26.9 us (5.6 TB/s, what whole tiles of the same bytes take), 29.0 by tiles.
+// NL chunks a thread; a chunk past the band loads its last row again.
+// row = id / cpr by multiplication: exact for id < 4096, as cpr < 32 keeps
+// id * (cpr * magic - 2^20) below 2^20.
+template <int DT, int CDT, int T, int NL>
+__device__ __forceinline__ void band_body(const Desc& d, int64_t b, int64_t r0, int64_t u, int pow2, int scale_bf16,
+                                          uint32_t (*red)[T / 64]) {
+  static_assert(DT != kF32 && NL * T <= 4096, "");
+  const int tid = threadIdx.x;
+  const uint32_t cpr = (uint32_t)d.cols >> 3, magic = (1u << 20) / cpr + 1;
+  const int last = (int)(d.rows - r0 < 128 ? d.rows - r0 : 128) - 1;
+  const int64_t in_base = b * d.bstride + r0 * d.ld;
+  Chunk<DT> ch[NL];
+#pragma unroll
+  for (int i = 0; i < NL; ++i) {
+    const uint32_t id = tid + T * i, row = id * magic >> 20, c = id - row * cpr;
+    load_chunk<DT>(ch[i], d.in, in_base + (int)(row < (uint32_t)last ? row : (uint32_t)last) * d.ld + 8 * c);
+  }
+  Amax<DT> am[2];
+  am[0].init();
+  am[1].init();
+#pragma unroll
+  for (int i = 0; i < NL; ++i) {
+    const uint32_t id = tid + T * i, c = id - (id * magic >> 20) * cpr;
+    Chunk<DT> lo = ch[i], hi = ch[i];
+#pragma unroll
+    for (int k = 0; k < Chunk<DT>::kWords; ++k) {
+      lo.w[k] = c < 16 ? lo.w[k] : 0u;
+      hi.w[k] = c < 16 ? 0u : hi.w[k];
+    }
+    am[0].add(lo);
+    am[1].add(hi);
+  }
+  const uint32_t a0 = group_max<64>(am[0].bits()), a1 = group_max<64>(am[1].bits());
+  if ((tid & 63) == 0) red[0][tid >> 6] = a0, red[1][tid >> 6] = a1;
+  __syncthreads();
+  BlockScale bs[2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    uint32_t a = red[t][0];
+#pragma unroll
+    for (int w = 1; w < T / 64; ++w) a = red[t][w] > a ? red[t][w] : a;
+    bs[t] = block_scale<CDT>(__builtin_amdgcn_readfirstlane(a), pow2 != 0);
+    if (tid == 0) store_scale<CDT>(d.scales, 2 * u + t, bs[t].s, scale_bf16);
+  }
+  uint8_t* const out = d.codes + (b * d.rows + r0) * d.cols;  // a band's rows are contiguous
+#pragma unroll
+  for (int i = 0; i < NL; ++i) {
+    const uint32_t id = tid + T * i, row = id * magic >> 20, c = id - row * cpr;
+    const BlockScale mine = c < 16 ? bs[0] : bs[1];
+    const v2u q = encode_chunk<DT, CDT>(ch[i], mine);
+    if (row <= (uint32_t)last) store_nt(out + 8 * id, q);
+  }
+}
+
 template <int DT, int CDT, int T>
 __global__ __launch_bounds__(T) void k_tile128(Desc single, const Desc* __restrict__ descs,
                                                const uint32_t* __restrict__ map, int pow2,
                                                int scale_bf16) {
-  __shared__ uint32_t red[T / 64];
+  __shared__ uint32_t red[2][T / 64];
   Desc d;
   int64_t u;
   pick_desc_tile(single, descs, map, d, u);
@@ -202,9 +261,15 @@ __global__ __launch_bounds__(T) void k_tile128(Desc single, const Desc* __restri
   const int64_t tr = rem / d.units_c;
   const int64_t tc = rem - tr * d.units_c;
   const int64_t r0 = tr * 128, c0 = tc * 128;
-  if (r0 + 128 <= d.rows && c0 + 128 <= d.cols) tile_body<DT, CDT, T, 16, true>(d, b, r0, c0, u, pow2, scale_bf16, red);
-  else if (d.cols - c0 > 64) tile_body<DT, CDT, T, 16, false>(d, b, r0, c0, u, pow2, scale_bf16, red);
-  else tile_body<DT, CDT, T, 8, false>(d, b, r0, c0, u, pow2, scale_bf16, red);
+  if constexpr (DT != kF32) {
+    if (d.units_c == 1 && d.cols > 128) {
+      band_body<DT, CDT, T, 6>(d, b, r0, u, pow2, scale_bf16, red);
+      return;
+    }
+  }
+  if (r0 + 128 <= d.rows && c0 + 128 <= d.cols) tile_body<DT, CDT, T, 16, true>(d, b, r0, c0, u, pow2, scale_bf16, red[0]);
+  else if (d.cols - c0 > 64) tile_body<DT, CDT, T, 16, false>(d, b, r0, c0, u, pow2, scale_bf16, red[0]);
+  else tile_body<DT, CDT, T, 8, false>(d, b, r0, c0, u, pow2, scale_bf16, red[0]);
 }
 
 // ---------------------------------------------------------------------------

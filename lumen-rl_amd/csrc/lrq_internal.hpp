@@ -18,7 +18,7 @@ struct Desc {
   int64_t batch, rows, cols, ld, bstride;
   int64_t unit0;
   int64_t units;     // work-groups of this tensor
-  int64_t units_c;   // tile kernel: tiles per row band; amax: 1 = 16-byte loads
+  int64_t units_c;   // tile kernel: tiles per row band (1: or both, tile_band); amax: 1 = 16-byte loads
   int64_t units_r;   // tile kernel: tile rows per matrix; amax: 1 = contiguous
   int64_t nblocks;   // row/MX kernels: number of blocks/groups
   int64_t bpr;       // row/MX kernels: blocks (groups) per row; k_tile128: log2 of its XCD run
@@ -97,6 +97,16 @@ constexpr int kTileRunLog2Wide = 2;    // rows of a multiple of 8 KiB: runs of 4
 constexpr int kTileRunLog2Narrow = 3;  // any other row pitch: runs of 8
 constexpr int tile_run_log2(int64_t pitch_bytes) {
   return pitch_bytes % 8192 == 0 ? kTileRunLog2Wide : kTileRunLog2Narrow;
+}
+// k_tile128: one work-group for both tiles of a row band (units_c = 1), for 16-bit
+// matrices of 136 to 192 columns with a band for each of the 256 CUs.  2048 x 192 by
+// 128: 26.9 us, 29.0 with a work-group per tile; x 176: 25.0 and 42.3; x 136: 20.6 and
+// 30.0; 256 bands of 136 columns 5.2 and 5.4.  Fewer bands leave CUs idle (64 bands of
+// 192 columns: 5.0 us, 4.5 per tile), and wider ones take registers that cost every
+// tile its eighth wave (76 for 8 chunks a thread, 52 for 6).
+constexpr int64_t kBandsMin = 256;
+constexpr bool tile_band(int dtype, int64_t cols, int64_t bands) {
+  return dtype != kF32 && cols > 128 && cols <= 192 && bands >= kBandsMin;
 }
 constexpr int64_t kXcdRunTileF64 = 32;  // k_tile_f64: 32 tiles (128 KiB each)
 constexpr int64_t kXcdRunRow = 16;     // k_row: 256 KiB of bf16 (32 loses 2%)

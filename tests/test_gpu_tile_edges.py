@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 import torch
 
-from lumenrl_amd.quantization import fp8_block_quant
+from lumenrl_amd.quantization import QuantPlan, fp8_block_quant
 from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -16,7 +16,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("rows", [1, 31, 127, 129, 200])
-@pytest.mark.parametrize("cols", [8, 56, 64, 72, 120, 128, 136, 192, 200, 264])
+@pytest.mark.parametrize("cols", [8, 56, 64, 72, 120, 128, 136, 144, 184, 192, 200, 264])
 def test_cut_tiles_vs_oracle(dtype, rows, cols):
     g = torch.Generator().manual_seed(rows * 1000 + cols)
     x = torch.randn(2, rows, cols + 8, generator=g) * 0.02
@@ -32,3 +32,24 @@ def test_cut_tiles_vs_oracle(dtype, rows, cols):
         oc, osc = O.fp8_block_quant(h, name, "f32", (128, 128))
         assert np.array_equal(codes[b].view(torch.uint8).cpu().numpy(), oc[0])
         assert np.array_equal(scales[b].cpu().numpy().view(np.uint32), osc[0].view(np.uint32))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("options", [{}, {"pow2": True}, {"scale_dtype": torch.bfloat16}, {"native_arith": True}])
+def test_bands_of_two_tiles_in_a_plan(dtype, options):
+    """Widths of 136 to 192 with 256 row bands or more, where one work-group makes both
+    tiles of a band (whole and cut ones, and one band too few), in one table with widths
+    that take a work-group per tile: each column of tiles as a call by itself gives it."""
+    g = torch.Generator().manual_seed(5)
+    shapes = [(86, 300, 192), (256, 128, 136), (300, 1, 176), (2, 256, 256), (52, 640, 184), (255, 40, 144), (1, 40, 64)]
+    xs = [(torch.randn(s, generator=g) * 0.02).to(dtype).cuda() for s in shapes]
+    xs[0][1, 130, 5], xs[0][2, 3, 150], xs[4][:, 600, 130] = float("nan"), float("inf"), 0.0
+    xs[4][3, :128] = 0.0
+    xs[4][5, 128:256, 128:] = torch.finfo(dtype).tiny
+    plan = QuantPlan(xs, "fp8_block", (128, 128), **{"use_pow2_scale" if k == "pow2" else k: v for k, v in options.items()})
+    for x, (codes, scales) in zip(xs, plan.run()):
+        codes, scales = codes.view(torch.uint8), scales.view(torch.uint8).view(*scales.shape, -1)
+        for c in range(0, x.shape[-1], 128):
+            tile, s = fp8_block_quant(x[..., c:c + 128].contiguous(), (128, 128), **options)
+            assert torch.equal(codes[..., c:c + 128], tile.view(torch.uint8))
+            assert torch.equal(scales[..., c // 128:c // 128 + 1, :], s.view(torch.uint8).view(*s.shape, -1))
