@@ -158,13 +158,14 @@ class FP8KVCacheQuantizer:
         for (short, module), (dt, i) in zip(targets, self._slots):
             name = _BUFFER_PREFIX + short
             buf = module._buffers.get(name)
-            if buf is None and hasattr(module, name):
+            there = buf is not None or hasattr(module, name)  # a failing look-up takes 1 us
+            if there and buf is None:
                 buf = getattr(module, name)
             at, dev = base[dt]
             if isinstance(buf, Tensor) and buf.data_ptr() == at + 4 * i and buf.device == dev:
                 continue  # a view of the vector the kernels have just written
             s = vecs[dt][i]
-            if name in module._buffers or hasattr(module, name):
+            if there:
                 buf.copy_(s.to(buf.device))
             else:
                 home = module.weight.device
