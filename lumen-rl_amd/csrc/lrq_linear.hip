@@ -17,10 +17,15 @@
 //     the whole block becomes NaN.  Such an x makes every output of its row inf
 //     or NaN here, so an output that is inf looks its operands over again
 //     (`linear_out`).
-//   * The block sums leave out the weight's scale, so they could overflow where
-//     y does not.  bf16 x is therefore multiplied with code * 2^-17 (exact in
-//     bf16), which bounds a block's sum by 2^127 for every finite x, and the
-//     result with 2^17; fp16 x cannot overflow a float32 sum.
+//   * x and code together are multiples of 2^-142, so the float32 block sums lose
+//     nothing to underflow: the matrix cores keep subnormals.
+//   * The block sums leave out the weight's scale, so with bf16 x beyond 2^112 they
+//     can overflow where y does not (fp16 x cannot).  A work-group that finds an inf
+//     or NaN among its results multiplies once more, with code * 2^-17 (exact in
+//     bf16, and every block's sum of finite x below 2^127), and takes those results,
+//     times 2^17, from there.  The others stay as they are: in units of 2^-17 all
+//     sums would come 17 binades nearer to underflow (with results of 2^-124, a
+//     relative error of 5.2e-3 instead of the rounding's 1.7e-3).
 #include "lrq.h"
 #include "lrq_device.hpp"
 #include "lrq_internal.hpp"
@@ -48,20 +53,29 @@ __device__ __forceinline__ float x16_to_f32(uint16_t b) {
 }
 
 // 8 codes (two words) as the matrix cores' second operand, in x's type: the
-// code itself (fp16) or 2^-17 times it (bf16), both exact.
+// code itself or, in the second pass that only bf16 has, 2^-17 times it.
 template <int DT>
-constexpr float kCodeUnit = DT == kBF16 ? 0x1p-17f : 1.0f;
-template <int DT, bool HI>
+constexpr bool kTwoPasses = DT == kBF16;
+constexpr float kSecondUnit = 0x1p-17f, kSecondResult = 0x1p17f;
+template <int DT, bool SECOND, bool HI>
 __device__ __forceinline__ uint32_t codes2_to_x16(uint32_t w) {
   if constexpr (DT == kBF16)
-    return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, kCodeUnit<DT>, HI));
+    return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, SECOND ? kSecondUnit : 1.0f, HI));
   else
-    return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w, kCodeUnit<DT>, HI));
+    return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w, 1.0f, HI));
 }
-template <int DT>
+template <int DT, bool SECOND>
 __device__ __forceinline__ v4u codes_to_x16(uint32_t lo, uint32_t hi) {
-  return v4u{codes2_to_x16<DT, false>(lo), codes2_to_x16<DT, true>(lo), codes2_to_x16<DT, false>(hi),
-             codes2_to_x16<DT, true>(hi)};
+  return v4u{codes2_to_x16<DT, SECOND, false>(lo), codes2_to_x16<DT, SECOND, true>(lo),
+             codes2_to_x16<DT, SECOND, false>(hi), codes2_to_x16<DT, SECOND, true>(hi)};
+}
+// The thread's index, which the second pass takes anew: offsets that it shared
+// with the first would be kept for it, in registers that the first has no more of.
+template <bool SECOND>
+__device__ __forceinline__ int linear_tid() {
+  int tid = threadIdx.x;
+  if constexpr (SECOND) asm volatile("" : "+v"(tid));
+  return tid;
 }
 
 // D[m][n] += sum over 32 k of A[m][k] B[k][n].  Lane l holds k = 8 (l / 16) ..
@@ -82,6 +96,26 @@ __device__ __forceinline__ void wave_lds_fence() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Barrier of the work-group for its LDS accesses only: loads from memory stay
+// in flight across it.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// True in every thread if any of the work-group's has `bad`; `flags`: a word of
+// LDS for each of its waves, free since the last barrier and until this returns.
+template <int WAVES>
+__device__ __forceinline__ bool linear_any(uint32_t* flags, bool bad) {
+  const uint32_t mine = __any(bad) ? 1u : 0u;
+  if ((threadIdx.x & 63) == 0) flags[threadIdx.x >> 6] = mine;
+  lds_barrier();
+  if (!__any((int)flags[threadIdx.x % WAVES])) return false;
+  lds_barrier();
+  return true;
 }
 
 // True if a row of x (k elements) or a weight row's scales hold an inf or NaN.
@@ -112,18 +146,24 @@ __device__ __forceinline__ uint16_t linear_bits(float v) {
   else return (uint16_t)f16_bits(v);
 }
 
-// y[m][n] from its sum (in units of kCodeUnit).  An inf is the sum's own
-// overflow, as in the reference, unless x's row or the scales are not finite:
-// the reference's ops give NaN there (x / inf * inf; a block scale of inf only
-// goes with NaN codes).
+__device__ __forceinline__ bool linear_finite(float v) { return (f2u(v) & 0x7FFFFFFFu) < 0x7F800000u; }
+template <int DT>
+__device__ __forceinline__ bool linear_bits_finite(uint16_t v) {
+  constexpr uint16_t kInf = DT == kBF16 ? 0x7F80u : 0x7C00u;
+  return (v & kInf) != kInf;
+}
+
+// y[m][n] from its sum; REDO: what is not finite is looked at in the second pass.
+// An inf is the sum's own overflow, as in the reference, unless x's row or the
+// scales are not finite: the reference's ops give NaN there (x / inf * inf; a
+// block scale of inf only goes with NaN codes).
 template <int DT>
 __device__ __forceinline__ bool linear_is_nan(const LinearArgs& a, int m, int n) {
   return linear_nonfinite<DT>(static_cast<const uint16_t*>(a.x) + m * a.ldx, a.scales + n * (a.k / kLinBlock), (int)a.k);
 }
-template <int DT>
+template <int DT, bool REDO>
 __device__ __forceinline__ uint16_t linear_out(const LinearArgs& a, float sum, int m, int n) {
-  sum *= 1.0f / kCodeUnit<DT>;
-  if ((f2u(sum) & 0x7FFFFFFFu) == 0x7F800000u && linear_is_nan<DT>(a, m, n)) sum = u2f(0x7FC00000u);
+  if (!REDO && (f2u(sum) & 0x7FFFFFFFu) == 0x7F800000u && linear_is_nan<DT>(a, m, n)) sum = u2f(0x7FC00000u);
   if (a.bias != nullptr) sum += linear_bias(a, n);
   return linear_bits<DT>(sum);
 }
@@ -161,13 +201,12 @@ struct LinStage {
   v4u x[MT][4];  // x: rows 4 i + lane / 16, 16-byte piece lane % 16
 };
 
-template <int DT, int MT, int NT, int KW, bool ONCE>
-__global__ __launch_bounds__(64 * KW) void k_linear_rows(LinearArgs a) {
+template <int DT, int MT, int NT, int KW, bool ONCE, bool SECOND>
+__device__ __forceinline__ bool linear_rows_pass(const LinearArgs& a, uint8_t* lds) {
   constexpr int COLS = 16 * NT, CELLS = 16 * MT * COLS;
   constexpr int kStageBytes = NT * 2048 + MT * 4096;
-  constexpr int kLds = KW * kStageBytes > KW * CELLS * 4 ? KW * kStageBytes : KW * CELLS * 4;
-  __shared__ __attribute__((aligned(16))) uint8_t lds[kLds];
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int tid = linear_tid<SECOND>();
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 15, g = lane >> 4;
   const int n0 = blockIdx.x * COLS, m0 = blockIdx.y * (16 * MT);
   const int n_last = (int)a.n - 1 - n0, m_last = (int)a.m - 1 - m0;  // within this tile
@@ -251,8 +290,8 @@ __global__ __launch_bounds__(64 * KW) void k_linear_rows(LinearArgs a) {
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         const v4u w = *reinterpret_cast<const v4u*>(lw + 2048 * j + 128 * c + 16 * ((g + 4 * h) ^ (c >> 1)));
-        b[2 * h] = codes_to_x16<DT>(w.x, w.y);
-        b[2 * h + 1] = codes_to_x16<DT>(w.z, w.w);
+        b[2 * h] = codes_to_x16<DT, SECOND>(w.x, w.y);
+        b[2 * h + 1] = codes_to_x16<DT, SECOND>(w.z, w.w);
       }
 #pragma unroll
       for (int i = 0; i < MT; ++i) {
@@ -288,14 +327,33 @@ __global__ __launch_bounds__(64 * KW) void k_linear_rows(LinearArgs a) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) red[wave * CELLS + (16 * i + 4 * g + r) * COLS + 16 * j + c] = acc[i][j][r];
   __syncthreads();
-  for (int e = threadIdx.x; e < CELLS; e += 64 * KW) {
+  bool bad = false;  // a result that the second pass replaces
+  for (int e = tid; e < CELLS; e += 64 * KW) {
     const int r = e / COLS, q = e % COLS;
     if (r > m_last || q > n_last) continue;
     float sum = red[e];
 #pragma unroll
     for (int w = 1; w < KW; ++w) sum += red[w * CELLS + e];
-    gst<uint16_t>(static_cast<uint16_t*>(a.y) + (int64_t)(m0 + r) * a.n + n0 + q, linear_out<DT>(a, sum, m0 + r, n0 + q));
+    uint16_t* const y = static_cast<uint16_t*>(a.y) + (int64_t)(m0 + r) * a.n + n0 + q;
+    if constexpr (SECOND) {
+      if (linear_bits_finite<DT>(gld<uint16_t>(y))) continue;  // what this thread stored in the first pass
+      sum *= kSecondResult;
+    } else if constexpr (kTwoPasses<DT>) {
+      bad |= !linear_finite(sum);
+    }
+    gst<uint16_t>(y, linear_out<DT, !SECOND && kTwoPasses<DT>>(a, sum, m0 + r, n0 + q));
   }
+  return bad;
+}
+
+template <int DT, int MT, int NT, int KW, bool ONCE>
+__global__ __launch_bounds__(64 * KW) void k_linear_rows(LinearArgs a) {
+  constexpr int kStages = KW * (NT * 2048 + MT * 4096), kSums = KW * (16 * MT) * (16 * NT) * 4;
+  static_assert(kSums + 4 * KW <= kStages, "the waves' sums and flags fit where their stages were");
+  __shared__ __attribute__((aligned(16))) uint8_t lds[kStages];
+  const bool bad = linear_rows_pass<DT, MT, NT, KW, ONCE, false>(a, lds);
+  if constexpr (kTwoPasses<DT>)
+    if (linear_any<KW>(reinterpret_cast<uint32_t*>(lds + kSums), bad)) linear_rows_pass<DT, MT, NT, KW, ONCE, true>(a, lds);
 }
 
 // ---------------------------------------------------------------------------
@@ -339,25 +397,18 @@ __device__ __forceinline__ void linear_tile(int wg, int tiles_m, int tiles_n, in
   tn = (t % group) / rows;
 }
 
-// Barrier of the work-group for its LDS accesses only: loads from memory stay
-// in flight across it.
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
-template <int DT, int FM, int FN, int WM, int WN>
-__global__ __launch_bounds__(64 * WM * WN, 1) void k_linear_tiles(LinearArgs a, int tiles_m, int tiles_n) {
+template <int FM, int FN, int WM, int WN>
+constexpr int kTileBuffer = 16 * FM * WM * 256 + 16 * FN * WN * (128 + 4);  // x, codes and scales of a K block
+template <int FM, int FN, int WM, int WN>
+constexpr int kTileResult = WM * WN * (16 * FM) * (2 * (16 * FN) + 16);  // y, by waves, in rows of a pitch
+template <int DT, int FM, int FN, int WM, int WN, bool SECOND>
+__device__ __forceinline__ bool linear_tiles_pass(const LinearArgs& a, int tm, int tn, uint8_t* lds) {
   constexpr int T = 64 * WM * WN, BM = 16 * FM * WM, BN = 16 * FN * WN;
   constexpr int PA = BM * 16 / T, PB = BN * 8 / T;   // 16-byte pieces a thread moves per K block
-  constexpr int kA = BM * 256, kB = BN * 128, kBuf = kA + kB + BN * 4;
+  constexpr int kA = BM * 256, kB = BN * 128, kBuf = kTileBuffer<FM, FN, WM, WN>;
   static_assert(BN <= T && PA * T == BM * 16 && PB * T == BN * 8, "");
-  __shared__ __attribute__((aligned(16))) uint8_t lds[2 * kBuf];
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tid = linear_tid<SECOND>(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 15, g = lane >> 4;
-  int tm, tn;
-  linear_tile(blockIdx.x, tiles_m, tiles_n, tm, tn);
   const int m0 = tm * BM, n0 = tn * BN;
   const int n_last = (int)a.n - 1 - n0, m_last = (int)a.m - 1 - m0;
   const int kb_n = (int)(a.k / kLinBlock);
@@ -465,7 +516,7 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void k_linear_tiles(LinearArgs a, 
       }
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const v4u b = (q & 1) ? codes_to_x16<DT>(w[q >> 1].z, w[q >> 1].w) : codes_to_x16<DT>(w[q >> 1].x, w[q >> 1].y);
+        const v4u b = (q & 1) ? codes_to_x16<DT, SECOND>(w[q >> 1].z, w[q >> 1].w) : codes_to_x16<DT, SECOND>(w[q >> 1].x, w[q >> 1].y);
 #pragma unroll
         for (int i = 0; i < FM; ++i) p[i] = mfma16<DT>(xa[i][q], b, q ? p[i] : f32x4{0.0f, 0.0f, 0.0f, 0.0f});
         if (j + 1 == FN) {
@@ -489,10 +540,11 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void k_linear_tiles(LinearArgs a, 
   // The wave's part of y goes through its own piece of LDS (no block is read
   // any more), so that rows leave in 16-byte stores.
   constexpr int ROWS = 16 * FM, COLS = 16 * FN, PITCH = 2 * COLS + 16, PIECES = COLS / 8;
-  static_assert(WM * WN * ROWS * PITCH <= 2 * kBuf, "the tile of y fits where the blocks were");
+  static_assert(WM * WN * ROWS * PITCH == kTileResult<FM, FN, WM, WN>, "");
   uint8_t* const out = lds + wave * (ROWS * PITCH);
+  constexpr bool kFirst = kTwoPasses<DT> && !SECOND;
   lds_barrier();
-  bool inf = false;
+  bool inf = false, bad = false;
 #pragma unroll
   for (int j = 0; j < FN; ++j) {
     const int n = wn + 16 * j + c;
@@ -501,8 +553,9 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void k_linear_tiles(LinearArgs a, 
     for (int i = 0; i < FM; ++i)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const float sum = acc[i][j][r] * (1.0f / kCodeUnit<DT>);
-        inf |= (f2u(sum) & 0x7FFFFFFFu) == 0x7F800000u;
+        const float sum = SECOND ? acc[i][j][r] * kSecondResult : acc[i][j][r];
+        if constexpr (kFirst) bad |= !linear_finite(sum);
+        else inf |= (f2u(sum) & 0x7FFFFFFFu) == 0x7F800000u;
         *reinterpret_cast<uint16_t*>(out + (16 * i + 4 * g + r) * PITCH + 2 * (16 * j + c)) = linear_bits<DT>(sum + bias);
       }
   }
@@ -524,12 +577,30 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void k_linear_tiles(LinearArgs a, 
     if (wm + m > m_last || n > n_last) continue;
     uint16_t* const dst = static_cast<uint16_t*>(a.y) + (int64_t)(m0 + wm + m) * a.n + n0 + n;
     const uint8_t* const src = out + m * PITCH + 16 * q;
-    if (whole) {
+    if (whole && !SECOND) {
       gst<v4u>(dst, *reinterpret_cast<const v4u*>(src));
     } else {
-      for (int k = 0; k < 8 && n + k <= n_last; ++k) gst<uint16_t>(dst + k, reinterpret_cast<const uint16_t*>(src)[k]);
+      for (int k = 0; k < 8 && n + k <= n_last; ++k) {
+        // the second pass replaces what this lane stored in the first where that is not finite
+        if (SECOND && linear_bits_finite<DT>(gld<uint16_t>(dst + k))) continue;
+        gst<uint16_t>(dst + k, reinterpret_cast<const uint16_t*>(src)[k]);
+      }
     }
   }
+  return bad;
+}
+
+template <int DT, int FM, int FN, int WM, int WN>
+__global__ __launch_bounds__(64 * WM * WN, 1) void k_linear_tiles(LinearArgs a, int tiles_m, int tiles_n) {
+  constexpr int kLds = 2 * kTileBuffer<FM, FN, WM, WN>, kResult = kTileResult<FM, FN, WM, WN>;
+  static_assert(kResult + 4 * WM * WN <= kLds, "the tile of y and the waves' flags fit where the blocks were");
+  __shared__ __attribute__((aligned(16))) uint8_t lds[kLds];
+  int tm, tn;
+  linear_tile(blockIdx.x, tiles_m, tiles_n, tm, tn);
+  const bool bad = linear_tiles_pass<DT, FM, FN, WM, WN, false>(a, tm, tn, lds);
+  if constexpr (kTwoPasses<DT>)
+    if (linear_any<WM * WN>(reinterpret_cast<uint32_t*>(lds + kResult), bad))
+      linear_tiles_pass<DT, FM, FN, WM, WN, true>(a, tm, tn, lds);
 }
 
 // ---------------------------------------------------------------------------

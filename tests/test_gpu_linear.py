@@ -32,11 +32,12 @@ def wide(codes, scales):
     return (codes.to(torch.float64).view(n, -1, 128) * scales.to(torch.float64)[..., None]).view(n, k)
 
 
-def check(y, x, codes, scales, bias=None):
+def check(y, x, codes, scales, bias=None, subnormal=2.0 ** -24):
     """|y - exact| within the result's own rounding and the float32 sums' bound:
     no sum is longer than 128 products, K/128 blocks and 16 waves or parts, each
     rounding (or truncating) by at most 2^-23 of the terms' magnitude; x_dq moves
-    a term by at most 2^-23 of itself."""
+    a term by at most 2^-23 of itself.  ``subnormal``: one unit of the type's
+    subnormals, twice their rounding."""
     k = x.shape[-1]
     w = wide(codes, scales)
     xd = x.double().reshape(-1, k)
@@ -44,7 +45,7 @@ def check(y, x, codes, scales, bias=None):
     if bias is not None:
         want, size = want + bias.double(), size + bias.double().abs()
     half_ulp = 2.0 ** -9 if y.dtype == torch.bfloat16 else 2.0 ** -12
-    bound = 2 * half_ulp * want.abs() + (128 + k // 128 + 20) * 2.0 ** -23 * size + 2.0 ** -24
+    bound = 2 * half_ulp * want.abs() + (128 + k // 128 + 20) * 2.0 ** -23 * size + subnormal
     off = (y.double() - want).abs()
     assert bool((off <= bound).all()), float((off / bound).max())
 
@@ -89,6 +90,35 @@ def test_linear_bias_strides_and_alignment(bias_dtype):
         fp8_linear(big[:1, :k].expand(3, k), codes, scales)
     with pytest.raises(ValueError):
         fp8_linear(big[:, :k], codes[:, :384], scales)
+
+
+# one shape for each kernel there is, its last rows and columns cut
+EVERY_KERNEL = [(15, 300), (5, 4099), (3, 8200), (31, 2170), (17, 4099), (30, 8200), (30, 12410), (40, 5510), (40, 8200),
+                (40, 1410), (60, 6275), (8200, 15), (70, 5510), (150, 4100), (200, 4100), (129, 12289), (390, 9364),
+                (1030, 6999)]
+
+
+@pytest.mark.parametrize("m,n", EVERY_KERNEL)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_linear_over_the_whole_exponent_range(dtype, m, n):
+    """Tokens from subnormal to near the type's maximum, in the same tiles: block sums that
+    overflow before the weight's scale is applied, results that are subnormal, and both in one
+    launch.  No token's result depends on another's size, or on another being inf or NaN."""
+    k = 384
+    _, codes, scales = operands(1, n, k, dtype, seed=m)
+    exps = [0, -112, 118, -118, 0, -124, 114, -130] if dtype == torch.bfloat16 else [0, -14, 10, -18, 0, -20, 11, -22]
+    g = torch.Generator(device=DEV).manual_seed(n)
+    x = torch.randn(m, k, generator=g, device=DEV).clamp(-4, 4).double()
+    x = (x * torch.tensor([2.0 ** exps[i % 8] for i in range(m)], device=DEV, dtype=torch.float64)[:, None]).to(dtype)
+    y = fp8_linear(x, codes, scales)
+    check(y, x, codes, scales, subnormal=2.0 ** -133 if dtype == torch.bfloat16 else 2.0 ** -24)
+    for bad in (float("inf"), float("nan")):
+        v = x.clone()
+        v[m // 2, 7] = bad
+        z = fp8_linear(v, codes, scales)
+        assert bool(z[m // 2].isnan().all())
+        z[m // 2] = y[m // 2]
+        assert torch.equal(z, y)
 
 
 @pytest.mark.parametrize("m,n", [(20, 272), (500, 4096), (1030, 7000)])  # each kernel
