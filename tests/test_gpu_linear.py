@@ -192,6 +192,55 @@ def test_module_routes(monkeypatch):
         check(y, x[0, :1].half(), half.weight_fp8, half.weight_scale)
 
 
+class _Watched(torch.Tensor):
+    seen = []
+
+    @classmethod
+    def __torch_function__(cls, func, types, args=(), kwargs=None):
+        cls.seen.append(func)
+        return super().__torch_function__(func, types, args, kwargs or {})
+
+
+def test_module_shows_its_linear_to_whoever_watches(monkeypatch):
+    """A function mode, a dispatch mode, a subclass of Tensor and the tracer see F.linear, as with
+    the library product; a default device, which is a function mode too, changes nothing."""
+    calls = []
+    real = ops.fp8_linear_checked
+    monkeypatch.setattr(ops, "fp8_linear_checked", lambda *a: calls.append(1) or real(*a))
+    torch.manual_seed(4)
+    mod, x = module(1024, 512, torch.bfloat16), torch.randn(5, 512, device=DEV, dtype=torch.bfloat16)
+    bias = mod.bias.detach()
+
+    class Functions(torch.overrides.TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            self.seen.append(func)
+            return func(*args, **(kwargs or {}))
+
+    class Operators(torch.utils._python_dispatch.TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.seen.append(func)
+            return func(*args, **(kwargs or {}))
+
+    with torch.no_grad():
+        y = mod(x)
+        assert calls == [1]
+        for mode in (Functions(), Operators()):
+            mode.seen = []
+            with mode:
+                check(mod(x), x, mod.weight_fp8, mod.weight_scale, bias)
+            assert any("linear" in str(f) or "addmm" in str(f) for f in mode.seen) and calls == [1]
+        with torch.device(DEV):
+            assert torch.equal(mod(x), y) and calls == [1, 1]
+        del mod.bias
+        mod.bias = bias.as_subclass(_Watched)
+        _Watched.seen.clear()
+        check(mod(x), x, mod.weight_fp8, mod.weight_scale, bias)
+        assert nn.functional.linear in _Watched.seen and calls == [1, 1]
+        mod.bias = bias
+        traced = torch.jit.trace(mod, (x,), check_trace=False)
+        assert "aten::linear" in str(traced.inlined_graph) and calls == [1, 1]
+
+
 def test_module_with_replaced_buffers():
     """A bias or scales that do not have one value per row (or block) of the weight
     go to the ops that check them: F.linear broadcasts one bias for all, and refuses
