@@ -93,12 +93,12 @@ def _projections(model: nn.Module) -> list[tuple[str, nn.Linear]]:
         for name, child in module._modules.items():
             if child is None:
                 continue
-            if type(child).named_modules is not nn.Module.named_modules:
+            if _own_traversal(child):
                 raise _OwnNames
             walk(child, name.rpartition(".")[2])
 
     try:
-        if type(model).named_modules is not nn.Module.named_modules:
+        if _own_traversal(model):
             raise _OwnNames
         walk(model, "")
     except _OwnNames:  # a module with a traversal of its own is asked for it
@@ -112,6 +112,13 @@ def _projections(model: nn.Module) -> list[tuple[str, nn.Linear]]:
 
 class _OwnNames(Exception):
     pass
+
+
+def _own_traversal(module) -> bool:
+    """True unless ``module.named_modules`` is nn.Module's: a class or an instance
+    may have its own, and a model may be a proxy that only delegates to a module."""
+    return (getattr(type(module), "named_modules", None) is not nn.Module.named_modules
+            or "named_modules" in module.__dict__)
 
 
 class FP8KVCacheQuantizer:
