@@ -260,16 +260,19 @@ def fp8_linear(x: Tensor, codes: Tensor, scales: Tensor, bias: Optional[Tensor] 
     if bias is not None and (tuple(bias.shape) != (n,) or bias.dtype not in _IN_DTYPES or bias.device != x.device
                              or not bias.is_contiguous()):
         raise ValueError(f"fp8_linear: bias must be a contiguous [{n}] tensor on {x.device}")
+    if k == 0:  # an empty sum
+        y = torch.zeros((_prod(x.shape[:-1]), n), dtype=torch.float32, device=x.device)
+        return (y if bias is None else y + bias).to(x.dtype)
     return fp8_linear_checked(x, codes, scales, bias)
 
 
 def fp8_linear_checked(x: Tensor, codes: Tensor, scales: Tensor, bias: Optional[Tensor]) -> Tensor:
-    """``fp8_linear`` of operands the caller has already checked."""
+    """``fp8_linear`` of operands the caller has already checked, K at least 128."""
     n, k = codes.shape
     if x.dim() == 2 and x.is_contiguous():
         xm, rows, ld = x, x.shape[0], k
     else:
-        rows = x.numel() // k if k else 0
+        rows = x.numel() // k
         xm = x.reshape(rows, k)
         if xm.stride(-1) != 1:  # as act_qdq: any row pitch and element alignment, but unit-stride rows
             xm = xm.contiguous()

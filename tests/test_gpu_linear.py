@@ -146,6 +146,17 @@ def test_linear_non_finite_and_extreme_values(dtype, m, n):
     assert bool(y[:, 5].isnan().all()) and not bool(y[:, 6:].isnan().any())
 
 
+@pytest.mark.parametrize("shape", [(0,), (3, 0), (2, 0, 0), (2, 5, 0)])
+def test_linear_of_no_columns(shape):
+    """K = 0: a row of the bias, or of zeros, for each token there is."""
+    x = torch.empty(shape, device=DEV, dtype=torch.bfloat16)
+    codes, scales = torch.empty(24, 0, device=DEV, dtype=torch.float8_e4m3fn), torch.empty(24, 0, device=DEV, dtype=torch.bfloat16)
+    bias = torch.randn(24, device=DEV)
+    rows = int(np.prod(shape[:-1]))
+    assert torch.equal(fp8_linear(x, codes, scales), torch.zeros(rows, 24, device=DEV, dtype=torch.bfloat16))
+    assert torch.equal(fp8_linear(x, codes, scales, bias), bias.bfloat16().expand(rows, 24))
+
+
 def module(out, cols, dtype, bias=True, blk=128):
     lin = nn.Linear(cols, out, bias=bias).to(DEV, dtype)
     cfg = FP8Config(precision="fp8")
