@@ -580,6 +580,23 @@ def test_fp8_linear_arguments_are_checked_before_any_device_call():
         assert call(**bad) == _lib.ERR_ALIGN, bad
 
 
+def test_fp8_linear_limits_are_those_of_the_python_side():
+    """At a limit the call gets as far as the alignment of x; past it, it does not."""
+    from lumenrl_amd.quantization import ops
+
+    fake, odd = ctypes.c_void_p(0x10000), ctypes.c_void_p(0x10001)
+
+    def call(rows=1, n=1, k=128, ld=128):
+        return L().lrq_fp8_linear(odd, 0, rows, k, ld, fake, fake, n, None, 0, fake, None)
+
+    tokens, out, pitch = ops.FP8_LINEAR_MAX_TOKENS, ops.FP8_LINEAR_MAX_OUT, ops.FP8_LINEAR_MAX_PITCH
+    cells = ops.FP8_LINEAR_MAX_CELLS // out
+    for inside, outside in (({"rows": tokens}, {"rows": tokens + 1}), ({"n": out}, {"n": out + 1}),
+                            ({"k": pitch, "ld": pitch}, {"k": pitch + 128, "ld": pitch + 128}),
+                            ({"ld": pitch}, {"ld": pitch + 1}), ({"rows": cells, "n": out}, {"rows": cells + 1, "n": out})):
+        assert call(**inside) == _lib.ERR_ALIGN and call(**outside) == _lib.ERR_ARG, inside
+
+
 def test_table_upload_checks_its_arguments_before_any_device_call():
     small, big = _pack(_lib.FMT_FP8_BLOCK, QWEN3_8B_LAYER), _pack(_lib.FMT_FP8_BLOCK, QWEN3_8B_LAYER * 5)
     dev = ctypes.c_void_p(0x1000)

@@ -194,3 +194,29 @@ def test_kv_quantizer_existing_buffers_cpu_model_and_disabled(caplog):
     with caplog.at_level(logging.WARNING):
         FP8KVCacheQuantizer(FP8Config(precision="fp8")).recalibrate_scales(nn.Sequential(nn.Linear(8, 8)))
     assert "no q_proj/k_proj/v_proj" in caplog.text
+
+
+def test_recalibrate_mixed_dtypes_twice():
+    """Projections of four types in turn, so that each scale's place in its type's group is
+    not its place in the model; twice, with new weights in place, and then with one moved."""
+    order = [torch.bfloat16, torch.float32, torch.float64, torch.float16, torch.float32, torch.bfloat16]
+    model, linears = nn.Sequential(), []
+    for i in range(4):
+        layer = nn.Module()
+        for j, name in enumerate(("v_proj", "q_proj", "k_proj")):
+            lin = nn.Linear(64 + 8 * i, 32 + 8 * j, bias=False, device=DEV, dtype=order[(5 * i + j) % 6])
+            layer.add_module(name, lin)
+            linears.append((lin, name))
+        model.append(layer)
+    kv = FP8KVCacheQuantizer(FP8Config(precision="fp8"))
+    for step in range(3):
+        with torch.no_grad():
+            for i, (lin, _) in enumerate(linears):
+                lin.weight.mul_(0.5).view(-1)[(7 * i + step) % lin.weight.numel()] = 1.0 + 0.125 * i + step
+            if step == 2:
+                linears[4][0].weight = nn.Parameter(linears[4][0].weight.clone())
+        kv.recalibrate_scales(model)
+        for i, (lin, name) in enumerate(linears):
+            got = getattr(lin, "_lumenrl_fp8_kv_scale_" + name)
+            amax = np.float32(lin.weight.detach().to(torch.float32).abs().max().item())
+            assert got.shape == () and bits(got) == int((amax / np.float32(448.0)).view(np.uint32)), (step, i)

@@ -4,6 +4,8 @@ product of the same codes, scales and activations, and the calls that
 
 from __future__ import annotations
 
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -50,7 +52,37 @@ def check(y, x, codes, scales, bias=None, subnormal=2.0 ** -24):
     assert bool((off <= bound).all()), float((off / bound).max())
 
 
-# tokens at the edges of the 16-row groups; weight rows at the edges of 16 to 64
+# one shape for each kernel there is, its last rows and columns cut
+EVERY_KERNEL = [(15, 300), (15, 4099), (15, 8200), (31, 2170), (17, 4099), (30, 8200), (30, 12410), (40, 5510), (40, 8200),
+                (40, 1410), (60, 6275), (8200, 15), (70, 5510), (150, 4100), (200, 4100), (129, 12289), (390, 9364),
+                (1030, 6999)]
+
+
+# K of one block, an odd number above the waves' eight, and two per wave
+@pytest.mark.parametrize("m,n", EVERY_KERNEL)
+@pytest.mark.parametrize("dtype,k", [(torch.bfloat16, 128), (torch.float16, 1152), (torch.bfloat16, 2048)])
+def test_linear_every_kernel_vs_float64(m, n, dtype, k):
+    x, codes, scales = operands(m, n, k, dtype, seed=m * 3 + n)
+    bias = torch.randn(n, device=DEV)
+    check(fp8_linear(x, codes, scales, bias), x, codes, scales, bias)
+
+
+@pytest.mark.parametrize("m,n", [(2, 4096), (48, 8200), (200, 4100), (1030, 6999)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_linear_rounds_its_sums_only(dtype, m, n):
+    """The share of results that are not the exact product's rounding.  Float32 sums over
+    K = 4096 are off by about 2e-6 of the result, which crosses a rounding boundary in 4e-6 of
+    a unit in the last place (2^-7 to 2^-8 of it in bf16, 2^-10 to 2^-11 in fp16): 0.1 % and
+    0.6 % at most, a few times that where terms cancel.  An operand rounded to bf16 is off by
+    1e-3: a third of the bf16 results, nearly all of the fp16 ones."""
+    k = 4096
+    x, codes, scales = operands(m, n, k, dtype, seed=11)
+    x[:, k // 3] /= 40.0
+    want = x.double() @ wide(codes, scales).T
+    assert (fp8_linear(x, codes, scales) != want.to(dtype)).double().mean() < 0.02
+
+
+# tokens at the edges of the 16-row groups; weight rows at the edges of 16 and 32
 # row tiles and where the tile's shape changes; K of fewer blocks than waves,
 # an odd number of blocks and several per wave
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
@@ -63,7 +95,7 @@ def test_linear_vs_float64(dtype, m, n, k):
     check(y, x, codes, scales)
 
 
-# many tokens: 64 x 128 and 128 x 256 tiles with whole and cut last rows and
+# many tokens: every size of tile, with whole and cut last rows and
 # columns (also widths that 8 does not divide, stored one by one), one block of K,
 # an odd number and an even one; grids of one round and of several
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
@@ -92,12 +124,6 @@ def test_linear_bias_strides_and_alignment(bias_dtype):
         fp8_linear(big[:, :k], codes[:, :384], scales)
 
 
-# one shape for each kernel there is, its last rows and columns cut
-EVERY_KERNEL = [(15, 300), (5, 4099), (3, 8200), (31, 2170), (17, 4099), (30, 8200), (30, 12410), (40, 5510), (40, 8200),
-                (40, 1410), (60, 6275), (8200, 15), (70, 5510), (150, 4100), (200, 4100), (129, 12289), (390, 9364),
-                (1030, 6999)]
-
-
 @pytest.mark.parametrize("m,n", EVERY_KERNEL)
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_linear_over_the_whole_exponent_range(dtype, m, n):
@@ -121,7 +147,7 @@ def test_linear_over_the_whole_exponent_range(dtype, m, n):
         assert torch.equal(z, y)
 
 
-@pytest.mark.parametrize("m,n", [(20, 272), (500, 4096), (1030, 7000)])  # each kernel
+@pytest.mark.parametrize("m,n", EVERY_KERNEL)
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_linear_non_finite_and_extreme_values(dtype, m, n):
     k = 512
@@ -212,6 +238,7 @@ class _Watched(torch.Tensor):
         return super().__torch_function__(func, types, args, kwargs or {})
 
 
+@pytest.mark.filterwarnings("ignore::torch.jit.TracerWarning")
 def test_module_shows_its_linear_to_whoever_watches(monkeypatch):
     """A function mode, a dispatch mode, a subclass of Tensor and the tracer see F.linear, as with
     the library product; a default device, which is a function mode too, changes nothing."""
@@ -281,6 +308,29 @@ def test_module_with_replaced_buffers():
         y = torch.vmap(with_bias)(batch)
         for i in range(3):
             check(y[i], x, codes, scales, batch[i])
+
+
+def test_linear_on_side_streams_from_two_threads():
+    """Each thread on a stream of its own, with inputs made there, many calls in flight."""
+    done = [None, None]
+
+    def work(i):
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            ops_ = [operands(m, 1100, 512, torch.bfloat16, seed=50 * i + m) for m in (1, 40, 200, 600)]
+            ys = [[fp8_linear(*o) for o in ops_] for _ in range(20)]
+        stream.synchronize()
+        done[i] = ops_, ys
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for ops_, ys in done:
+        for i, o in enumerate(ops_):
+            check(ys[0][i], *o)
+            assert all(torch.equal(y[i], ys[0][i]) for y in ys)
 
 
 def test_linear_in_a_graph():

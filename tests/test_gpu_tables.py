@@ -1,5 +1,5 @@
 """A device table written by one launch (lrq_group_upload) against the same table
-copied and mapped in two steps, byte for byte: one tensor, empty tensors first,
+copied and mapped in two steps, byte for byte but for padding: one tensor, empty tensors first,
 between and last, and as many tensors as the launch's arguments hold."""
 
 from __future__ import annotations
@@ -43,5 +43,7 @@ def test_one_launch_table_equals_copy_and_map(fmt, block, shapes):
     host[:] = 0  # the call keeps nothing of the host table
     torch.cuda.synchronize()
     one, two = one.cpu().numpy(), two.cpu().numpy()
-    gaps = one != two  # only padding, which nothing reads, is left unwritten
-    assert not gaps[256:256 + 112 * len(shapes)].any() and not gaps[need:].any() and (one[gaps] == 0xA5).all()
+    gaps = one != two  # only padding, which nothing reads, is left unwritten: behind the header and the descriptors
+    header, first, each = 104, 256, 112
+    assert not gaps[:header].any() and not gaps[first:first + each * len(shapes)].any()
+    assert not gaps[need:].any() and (one[gaps] == 0xA5).all()
