@@ -26,7 +26,7 @@ struct Desc {
 static_assert(sizeof(Desc) == 112, "Desc layout is part of the grouped table format");
 
 enum Kernel : int {
-  kKernTile128 = 0,   // 128x128 FP8 tiles, one work-group per tile
+  kKernTile128 = 0,   // 128x128 FP8 tiles, one work-group per tile (or per row band of two: tile_band)
   kKernRowQuad = 1,   // 1xB FP8 blocks, B/8 consecutive lanes per block
   kKernGenericFp8 = 2,
   kKernMx = 3,        // MXFP8 / MXFP4, one quad per 32-group

@@ -33,7 +33,6 @@
 namespace lrq {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
@@ -614,7 +613,9 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void k_linear_tiles(LinearArgs a, 
 //     tiles, three fit a CU, 280 ns and 457 once where they do.
 // From sweeps over all shapes at 1 to 8192 tokens and weights of [500 to 12288,
 // 1024 to 12288], where the shape it takes is 1 % from the fastest in the mean.
-constexpr int kLinearRows[3][4] = {{136, 190, 315, 380}, {165, 280, 400, 465}, {290, 380, 485, INT32_MAX}};
+// 16 tokens x 64 weight rows are left out (two rounds of 16 x 32 cost no more), and
+// 48 x 64 (more registers than there are).
+constexpr int kLinearRows[3][4] = {{136, 190, 315, 0}, {165, 280, 400, 465}, {290, 380, 485, 0}};
 struct LinearTile {
   int m, n, each, once;
 };
@@ -638,7 +639,7 @@ static LinearShape linear_shape(int64_t m, int64_t n) {
   }
   for (int mt = 1; mt <= 3 && 16 * (mt - 1) < m; ++mt) {
     if (ceil_div(m, 16 * mt) > 65535) continue;  // the grid's second dimension
-    for (int nt = 1; nt <= (mt < 3 ? 4 : 3); ++nt) {
+    for (int nt = 1; nt <= 4 && kLinearRows[mt - 1][nt - 1] > 0; ++nt) {
       const int64_t cost = kLinearRows[mt - 1][nt - 1] * ceil_div(ceil_div(n, 16 * nt) * ceil_div(m, 16 * mt), 256);
       if (cost < least) least = cost, best = {-1, mt, nt};
     }
@@ -650,8 +651,11 @@ template <int DT, int MT, int NT>
 static void launch_rows(const LinearArgs& a, hipStream_t stream) {
   constexpr int KW = 8;  // their LDS, 2 KiB per 16 weight rows and 4 per 16 tokens each, fits the CU's 160 KiB
   const dim3 grid((unsigned)ceil_div(a.n, 16 * NT), (unsigned)ceil_div(a.m, 16 * MT)), block(64 * KW);
-  if (grid.y == 1) hipLaunchKernelGGL((k_linear_rows<DT, MT, NT, KW, true>), grid, block, 0, stream, a);
-  else hipLaunchKernelGGL((k_linear_rows<DT, MT, NT, KW, false>), grid, block, 0, stream, a);
+  // One token group never takes 48 x 16 (32 x 32 costs less for the same rounds), and
+  // several never 16 x 48: ONCE is a hint for the caches, so neither needs the other kernel.
+  constexpr bool kOne = !(MT == 3 && NT == 1), kMany = !(MT == 1 && NT == 3);
+  if (kOne && (grid.y == 1 || !kMany)) hipLaunchKernelGGL((k_linear_rows<DT, MT, NT, KW, kOne>), grid, block, 0, stream, a);
+  else hipLaunchKernelGGL((k_linear_rows<DT, MT, NT, KW, !kMany>), grid, block, 0, stream, a);
 }
 template <int DT, int MT>
 static void launch_rows_nt(const LinearArgs& a, int nt, hipStream_t stream) {
@@ -660,7 +664,7 @@ static void launch_rows_nt(const LinearArgs& a, int nt, hipStream_t stream) {
     case 2: return launch_rows<DT, MT, 2>(a, stream);
     case 3: return launch_rows<DT, MT, 3>(a, stream);
     default:
-      if constexpr (MT < 3) launch_rows<DT, MT, 4>(a, stream);
+      if constexpr (MT == 2) launch_rows<DT, MT, 4>(a, stream);
   }
 }
 template <int DT, int FM, int FN, int WM, int WN>
