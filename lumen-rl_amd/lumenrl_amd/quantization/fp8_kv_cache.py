@@ -82,24 +82,23 @@ def _projections(model: nn.Module) -> list[tuple[str, nn.Linear]]:
     """(last name component, module) of every q/k/v projection, in the order and
     with the names of ``model.named_modules()``: each module once, under the
     first path that reaches it."""
-    found, seen = [], set()
+    found, seen, usual = [], set(), nn.Module.named_modules
 
     def walk(module: nn.Module, short: str) -> None:
+        # a class or an instance may have its own traversal, and a model may be a
+        # proxy that only delegates to a module
+        if getattr(type(module), "named_modules", None) is not usual or "named_modules" in module.__dict__:
+            raise _OwnNames
         if module in seen:
             return
         seen.add(module)
         if short in _KV_PROJECTIONS and isinstance(module, nn.Linear):
             found.append((short, module))
         for name, child in module._modules.items():
-            if child is None:
-                continue
-            if _own_traversal(child):
-                raise _OwnNames
-            walk(child, name.rpartition(".")[2])
+            if child is not None:
+                walk(child, name.rpartition(".")[2] if "." in name else name)
 
     try:
-        if _own_traversal(model):
-            raise _OwnNames
         walk(model, "")
     except _OwnNames:  # a module with a traversal of its own is asked for it
         found = []
@@ -112,13 +111,6 @@ def _projections(model: nn.Module) -> list[tuple[str, nn.Linear]]:
 
 class _OwnNames(Exception):
     pass
-
-
-def _own_traversal(module) -> bool:
-    """True unless ``module.named_modules`` is nn.Module's: a class or an instance
-    may have its own, and a model may be a proxy that only delegates to a module."""
-    return (getattr(type(module), "named_modules", None) is not nn.Module.named_modules
-            or "named_modules" in module.__dict__)
 
 
 class FP8KVCacheQuantizer:
