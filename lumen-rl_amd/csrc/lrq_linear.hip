@@ -25,7 +25,9 @@
 //     bf16, and every block's sum of finite x below 2^127), and takes those results,
 //     times 2^17, from there.  The others stay as they are: in units of 2^-17 all
 //     sums would come 17 binades nearer to underflow (with results of 2^-124, a
-//     relative error of 5.2e-3 instead of the rounding's 1.7e-3).
+//     relative error of 5.2e-3 instead of the rounding's 1.7e-3).  Such work-groups
+//     take twice as long: 8192 tokens x [12288, 4096] 1.18 ms with one inf and 1.55
+//     with NaN in every token (0.80 without), 48 tokens 34 us (18).
 #include "lrq.h"
 #include "lrq_device.hpp"
 #include "lrq_internal.hpp"
@@ -172,9 +174,9 @@ __device__ __forceinline__ uint16_t linear_out(const LinearArgs& a, float sum, i
 // ---------------------------------------------------------------------------
 // The weight's e4m3 bytes are all that has to move; dequantizing it to float32
 // for a library product wrote and read 8 times as many.  On an MI355X, one token
-// through a 4096 x 4096 weight takes 6.6 us (48 us a call before) and 48 tokens
-// through 12288 x 4096 17.2 us (105 us), where the weight's bytes alone take
-// 2.5 and 7.6 us: at few work-groups per CU the rest is latency, and from about
+// through a 4096 x 4096 weight takes 6.3 us (48 us a call before) and 48 tokens
+// through 12288 x 4096 18.8 us (105 us), medians of rocprofv3 traces, where the
+// weight's bytes alone take 2.5 and 7.6 us: at few work-groups per CU the rest is latency, and from about
 // 32 tokens on x's passage through each CU's cache and LDS.
 //
 // A work-group of KW waves makes a (16 MT) x (16 NT) tile of y over the whole
@@ -372,9 +374,10 @@ __global__ __launch_bounds__(64 * KW) void k_linear_rows(LinearArgs a) {
 // 4 x 4 x (2 x 4): 128 x 256 tiles, one work-group of 8 waves on a CU, two to a
 // SIMD, so that one's vector instructions and waits fall beside the other's
 // matrix instructions (4 waves of 128 x 64 each: 0.90 ms instead of 0.80).
-// 8192 tokens x [12288, 4096] take 0.79 ms (1046 TFLOP/s, matrix cores 47 % busy
-// at 1.9 GHz), 5.6 ms before by way of float32 operands and a float32 library
-// product (147 TFLOP/s).
+// 8192 tokens x [12288, 4096] take 0.80 ms (1032 TFLOP/s), 5.6 ms before by way of
+// float32 operands and a float32 library product (147 TFLOP/s).  That is 1.67 million
+// cycles, at 2.1 GHz: matrix cores busy 47 % of them, other vector instructions 35 %,
+// LDS 33 % (rocprofv3 counters; a profiled pass runs at a lower clock, 0.82 to 1.03 ms).
 // The smaller tiles are for grids that would leave CUs idle with the large one:
 // each CU does less work per byte that passes its LDS, 28 us for 512 tokens x
 // [4096, 4096] in 64 x 128 tiles (59 in 128 x 256), 115 us for 1024 x [12288,
@@ -611,11 +614,14 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void k_linear_tiles(LinearArgs a, 
 //     has two bytes an element); shapes past 8 waves' LDS do not pay any more;
 //   * k_linear_tiles: `each` ns for each 256 tiles, and `once` more; of 64 x 64
 //     tiles, three fit a CU, 280 ns and 457 once where they do.
-// From sweeps over all shapes at 1 to 8192 tokens and weights of [500 to 12288,
-// 1024 to 12288], where the shape it takes is 1 % from the fastest in the mean.
+// A sweep of every shape over 1 to 8192 tokens and weights of [512 to 12288, 1024 to
+// 12288], 197 sizes: the shape this takes is 1.1 % from the fastest in the mean, over
+// 5 % in 16 of them, and 31 % at worst (32 tokens x [2560, 2560] in 32 x 16: 6.7 us,
+// 5.1 in 16 x 32; one round of work-groups is charged the same however full it is).
 // 16 tokens x 64 weight rows are left out (two rounds of 16 x 32 cost no more), and
 // 48 x 64 (more registers than there are).
 constexpr int kLinearRows[3][4] = {{136, 190, 315, 0}, {165, 280, 400, 465}, {290, 380, 485, 0}};
+constexpr int64_t kCus = 256;
 struct LinearTile {
   int m, n, each, once;
 };
@@ -632,7 +638,7 @@ static LinearShape linear_shape(int64_t m, int64_t n) {
   int64_t least = INT64_MAX;
   for (int i = 0; i < kLinearTileKinds; ++i) {
     const LinearTile& t = kLinearTiles[i];
-    const int64_t rounds = ceil_div(ceil_div(m, t.m) * ceil_div(n, t.n), 256);
+    const int64_t rounds = ceil_div(ceil_div(m, t.m) * ceil_div(n, t.n), kCus);
     int64_t cost = t.each * rounds + t.once;
     if (t.m == 64 && t.n == 64 && 280 * rounds + 457 > cost) cost = 280 * rounds + 457;
     if (cost < least) least = cost, best = {i, 0, 0};
@@ -640,7 +646,7 @@ static LinearShape linear_shape(int64_t m, int64_t n) {
   for (int mt = 1; mt <= 3 && 16 * (mt - 1) < m; ++mt) {
     if (ceil_div(m, 16 * mt) > 65535) continue;  // the grid's second dimension
     for (int nt = 1; nt <= 4 && kLinearRows[mt - 1][nt - 1] > 0; ++nt) {
-      const int64_t cost = kLinearRows[mt - 1][nt - 1] * ceil_div(ceil_div(n, 16 * nt) * ceil_div(m, 16 * mt), 256);
+      const int64_t cost = kLinearRows[mt - 1][nt - 1] * ceil_div(ceil_div(n, 16 * nt) * ceil_div(m, 16 * mt), kCus);
       if (cost < least) least = cost, best = {-1, mt, nt};
     }
   }
